@@ -1,4 +1,5 @@
-// fp32 GEMM on CDNA4 matrix cores (v_mfma_f32_32x32x2_f32), LDS-staged tiles.
+// fp32 GEMM on CDNA4 matrix cores, small shapes (v_mfma_f32_32x32x2_f32), and
+// the choice of kernel for every shape.
 //
 // Replaces the reference's three CPU kernels (midman-tensor/src/kernels.rs:49-108,
 // kernels_avx.rs:45-250): C = A.B (nn), A.B^T (nt) and A^T.B (tn). The
@@ -6,382 +7,28 @@
 // kernels.rs:68-73): each operand is read in its stored layout and written into
 // LDS k-major, the layout the MFMA operand reads want.
 //
-// Tiling: a 512-thread workgroup (8 wave64s, 4 along M x 2 along N) owns a
-// 128x128 tile of C; each wave owns 32 rows x 64 columns as two MFMA 32x32
-// blocks (32 accumulators per lane), whose columns are the even and the odd
-// columns of its 64: one 4-byte A read and one 8-byte B read from LDS give a
-// lane its operands for both blocks, and the epilogue writes column pairs.
-// Eight small waves rather than four of 64x64 keep four waves on every SIMD
-// when a grid has only two tiles per CU (the O and down projections of the
-// large preset: 512 tiles), at under 110 registers. For the QKV product with
-// RoPE in the epilogue the column blocks instead hold columns c and c + hd/2
-// of a head (hd 64 or 128), so each rotation pair sits in one lane.
+// The products with enough 128x128 tiles of work run on gemm_split.hip's
+// kernels. Here are the 64x64 tiles (a workgroup each, one 32x32 MFMA block
+// per wave) and the 32x32 K-split tiles for the shapes that are bound by
+// latency rather than by the matrix cores' rate.
 //
 // MFMA 32x32x2 f32 operand layout (wave64): lane l supplies A[i=l%32][k=l/32]
 // and B[k=l/32][j=l%32]; accumulator register r of lane l holds
 // D[i = 8*(r/4) + 4*(l/32) + r%4][j = l%32].
-//
-// K advances 16 at a time through two LDS stages, software-pipelined: at the
-// top of iteration t, tile t+1 moves from registers into the free stage and
-// tile t+4's global loads are issued into the register slot it freed (a ring
-// of three slots); then the 16 MFMAs per wave of tile t run while the loads
-// of three tiles are in flight. One barrier per tile. Interior tiles take a
-// path with no load predicates and 32-bit offsets from uniform base
-// pointers; edge tiles zero-fill outside [M, N, K) and keep one slot.
-//
-// Workgroup -> tile mapping is XCD-aware: the dispatcher hands workgroup w to
-// XCD w % 8, so w is renumbered to make each XCD's share a contiguous run of
-// tiles, and tiles are walked in groups of 8 tile-rows so that the tiles an
-// XCD holds at once share A rows and B columns in its L2.
 //
 // Small-tile-count shapes (e.g. M=2048, N=256) are split along K; the
 // partials are summed in split order, so the result is deterministic: on the
 // 64x64 and 32x32 tiles by the last split of each tile (the splits store
 // their partial through to memory and count themselves in a per-tile
 // counter), on the 128x128 tiles by a second kernel.
-#include "mmh_internal.h"
+#include "mmh_gemm.h"
 
-#include <utility>
+#include <algorithm>
+#include <cmath>
 
 namespace mmh {
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
-constexpr int BM = 128, BN = 128, BK = 16;
-constexpr int NT = 512;  // threads of the 128x128 kernel: 8 waves
-constexpr int GROUP_M = 8;
-// Register slots of the 128x128 kernel's load ring on interior tiles: tile
-// t+KSLOTS's global loads are issued while tile t's MFMAs run. Edge tiles
-// (predicated loads, few per grid) keep one slot, which holds the kernel's
-// registers to what the interior path needs.
-constexpr int KSLOTS = 3;
-// Raw buffer descriptor: byte range (interior tiles stay below 2^31 bytes from
-// their base, checked on the host) and the gfx9-family dword-3 flags.
-constexpr int kBufferRange = 0x7fffffff;
-constexpr int kBufferFlags = 0x00020000;
-
-struct KParams {
-    const float *a;
-    const float *b;
-    float *c;
-    float *partial;
-    int64_t m, n, k;
-    int64_t lda, ldb, ldc;
-    int64_t stride_a, stride_b, stride_c;
-    int64_t k_per_split;
-    int64_t swiglu_ff;
-    const float *resid;
-    float *aux;
-    int64_t ldaux;
-    int tiles_m, tiles_n;
-    int splits;
-    int vec_a, vec_b, vec_c;
-    // small kernel only: A-row RMSNorm in the loads, RoPE in the epilogue
-    const float *norm_w;
-    float norm_eps;
-    const float *rope_cos, *rope_sin;
-    int rope_seq, rope_hd, rope_cols;
-    // EPI_CE (128x128 kernel): targets in, per-tile (max, sum) pairs and target logits out
-    const int32_t *ce_targets;
-    float *ce_part, *ce_zt;
-    // Tail balance (128x128 kernel, one matrix): workgroups from tail_first on
-    // each take one of tail_s K-pieces (tail_k long) of tiles tail_first.. in
-    // the grouped order, and write their partial tile to partial (tile-local
-    // [BM][BN] blocks, piece-major); tail_reduce sums them in piece order.
-    int tail_first, tail_s;
-    int64_t tail_k;
-    // Split K on the 64x64 and 32x32 tiles (tickets set): every split stores
-    // its partial tile through to memory and counts itself in tickets[tile];
-    // the last split of a tile sums the tile's partials in split order and
-    // applies the epilogue (split_accum: C = resid (or C) + sum, else C = sum).
-    int32_t *tickets;
-    int split_accum;
-    // The value the sums of products start from: +0 (a product, as the
-    // reference's fresh zeroed C), or -0 when the sum is added into C (the
-    // seam's accumulate: C's own value starts the reference's sum, so a -0 in
-    // C with all products -0 must stay -0; -0 is the identity of IEEE addition)
-    float acc_init;
-};
-
-// Row strides (floats) of the k-major LDS stages: even, so the 8-byte operand
-// reads stay aligned; +2 where the stores transpose (spreads consecutive k rows
-// over the banks), +4 where they are float4 (keeps 16-byte alignment).
-template <bool TA>
-struct LdsA {
-    static constexpr int S = BM + (TA ? 4 : 2);
-};
-template <bool TB>
-struct LdsB {
-    static constexpr int S = BN + (TB ? 2 : 4);
-};
-
-// Calls f(integral_constant<int, i>) for i = 0..n-1, so that i is a
-// compile-time constant in each call (register-slot indices stay static).
-template <class F, int... Is>
-__device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, Is...>) {
-    (f(std::integral_constant<int, Is>{}), ...);
-}
-
-// Reductions over each 32-lane half of a wave with DPP moves (quad permutes,
-// then rotations within a 16-lane row) and one v_permlane16_swap across the
-// two rows of the half (a VALU exchange: no trip through the LDS unit). For the max every lane ends with the result; for the sum the
-// lanes associate the terms differently, and lane 0 of the half (the one read)
-// always the same way.
-__device__ __forceinline__ float dpp_f(float v, int ctrl) {
-    switch (ctrl) {
-        case 0xB1: return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));
-        case 0x4E: return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false));
-        case 0x124: return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xF, 0xF, false));
-        default: return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xF, 0xF, false));
-    }
-}
-// The pair {v[l], v[l ^ 16]} in each lane l (in some order).
-__device__ __forceinline__ auto pair16_f(float v) {
-    return __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-}
-__device__ __forceinline__ float half_max32(float v) {
-    v = fmaxf(v, dpp_f(v, 0xB1));   // quad_perm [1,0,3,2]
-    v = fmaxf(v, dpp_f(v, 0x4E));   // quad_perm [2,3,0,1]
-    v = fmaxf(v, dpp_f(v, 0x124));  // row_ror:4
-    v = fmaxf(v, dpp_f(v, 0x128));  // row_ror:8
-    const auto q = pair16_f(v);
-    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
-}
-__device__ __forceinline__ float half_sum32(float v) {
-    v += dpp_f(v, 0xB1);
-    v += dpp_f(v, 0x4E);
-    v += dpp_f(v, 0x124);
-    v += dpp_f(v, 0x128);
-    const auto q = pair16_f(v);
-    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
-}
-
-// The K loop of one 128x128 tile; see the file comment.
-// CL: the columns of a wave's two MFMA column blocks: 0 the even and odd
-// columns of its 64 (one 8-byte operand read), 1 its two halves of 32, 2
-// columns c and c + 64 of the tile (wave wn takes c = 32*wn .. +31), so the
-// RoPE pair (c, c + hd/2) of a head of 64 (CL 1) or 128 (CL 2) columns sits
-// in one lane.
-template <bool TA, bool TB, bool FAST, int SLOTS, int CL, bool OPQ = false>
-__device__ __forceinline__ void gemm_mainloop(const KParams &p, const float *__restrict__ A,
-                                              const float *__restrict__ B, int64_t m0, int64_t n0,
-                                              int64_t kbeg, int64_t kend,
-                                              float (*As)[BK][LdsA<TA>::S],
-                                              float (*Bs)[BK][LdsB<TB>::S],
-                                              floatx16 (&acc)[2]) {
-    // OPQ: the thread index through an empty asm. The register assignment
-    // and schedule the compiler then picks ran the residual-epilogue forms
-    // 0.8-1.4% faster on the large forward's o and down products, and the
-    // SwiGLU and loss forms 2% slower, so only the former take it.
-    int tid = threadIdx.x;
-    if constexpr (OPQ) asm volatile("" : "+v"(tid));
-    const int64_t M = p.m, N = p.n;
-    // A K-tile of each operand is 128 x BK floats = 32*BK float4; thread tid
-    // moves float4 idx = tid + NT*i, i < NL.
-    // Row-major-in-k operands (A for nn/nt, B for nt): row idx/(BK/4), k (idx%(BK/4))*4.
-    // k-major operands (A for tn, B for nn/tn): k idx/32, column (idx%32)*4.
-    constexpr int NL = 32 * BK / NT;
-    static_assert(NL >= 1 && 32 * BK % NT == 0, "a K-tile must split evenly over the threads");
-    constexpr int RQ = BK / 4;  // float4 per row of a row-major-in-k tile
-    // Uniform bases (moved by the tile's k) and loop-invariant 32-bit byte
-    // offsets per thread, so each load is one SGPR base + VGPR offset
-    // instruction with no per-iteration address registers.
-    const float *a_base = TA ? A + m0 : A + m0 * p.lda;
-    const float *b_base = TB ? B + n0 * p.ldb : B + n0;
-    const uint32_t lda = (uint32_t)p.lda, ldb = (uint32_t)p.ldb;
-    uint32_t ao[NL], bo[NL];
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const int idx = tid + NT * i;
-        ao[i] = 4u * (TA ? (uint32_t)(idx >> 5) * lda + (idx & 31) * 4
-                         : (uint32_t)(idx / RQ) * lda + (idx % RQ) * 4);
-        bo[i] = 4u * (TB ? (uint32_t)(idx / RQ) * ldb + (idx % RQ) * 4
-                         : (uint32_t)(idx >> 5) * ldb + (idx & 31) * 4);
-    }
-
-    constexpr int NS = FAST ? SLOTS : 1;
-    float4 ra[NS][NL], rb[NS][NL];
-
-    // Values outside [M, N, K) read as zeros; A's are -0, so a product of two
-    // of them is -0, the identity of IEEE addition (a +0 would turn an exact
-    // -0 sum into +0).
-    auto load_a_edge = [&](int idx, int64_t k0) __attribute__((always_inline)) -> float4 {
-        float4 v = make_float4(-0.f, -0.f, -0.f, -0.f);
-        if (!TA) {
-            const int64_t gm = m0 + idx / RQ, gk = k0 + (idx % RQ) * 4;
-            if (gm < M) {
-                const float *src = A + gm * p.lda + gk;
-                if (gk + 0 < kend) v.x = src[0];
-                if (gk + 1 < kend) v.y = src[1];
-                if (gk + 2 < kend) v.z = src[2];
-                if (gk + 3 < kend) v.w = src[3];
-            }
-        } else {
-            const int64_t gk = k0 + (idx >> 5), gm = m0 + (idx & 31) * 4;
-            if (gk < kend) {
-                const float *src = A + gk * p.lda + gm;
-                if (gm + 0 < M) v.x = src[0];
-                if (gm + 1 < M) v.y = src[1];
-                if (gm + 2 < M) v.z = src[2];
-                if (gm + 3 < M) v.w = src[3];
-            }
-        }
-        return v;
-    };
-    auto load_b_edge = [&](int idx, int64_t k0) __attribute__((always_inline)) -> float4 {
-        float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (!TB) {
-            const int64_t gk = k0 + (idx >> 5), gn = n0 + (idx & 31) * 4;
-            if (gk < kend) {
-                const float *src = B + gk * p.ldb + gn;
-                if (gn + 0 < N) w.x = src[0];
-                if (gn + 1 < N) w.y = src[1];
-                if (gn + 2 < N) w.z = src[2];
-                if (gn + 3 < N) w.w = src[3];
-            }
-        } else {
-            const int64_t gn = n0 + idx / RQ, gk = k0 + (idx % RQ) * 4;
-            if (gn < N) {
-                const float *src = B + gn * p.ldb + gk;
-                if (gk + 0 < kend) w.x = src[0];
-                if (gk + 1 < kend) w.y = src[1];
-                if (gk + 2 < kend) w.z = src[2];
-                if (gk + 3 < kend) w.w = src[3];
-            }
-        }
-        return w;
-    };
-    auto load = [&](int sl, int64_t k0) __attribute__((always_inline)) {
-        if (FAST) {
-            // Buffer loads: the tile's base in a scalar descriptor, the
-            // per-thread byte offset in one loop-invariant VGPR.
-            const float *ak = TA ? a_base + k0 * p.lda : a_base + k0;
-            const float *bk = TB ? b_base + k0 : b_base + k0 * p.ldb;
-            const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float *>(ak), (short)0, kBufferRange, kBufferFlags);
-            const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float *>(bk), (short)0, kBufferRange, kBufferFlags);
-#pragma unroll
-            for (int i = 0; i < NL; ++i)
-                ra[sl][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsa, ao[i], 0, 0));
-#pragma unroll
-            for (int i = 0; i < NL; ++i)
-                rb[sl][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsb, bo[i], 0, 0));
-        } else {
-#pragma unroll
-            for (int i = 0; i < NL; ++i) ra[sl][i] = load_a_edge(tid + NT * i, k0);
-#pragma unroll
-            for (int i = 0; i < NL; ++i) rb[sl][i] = load_b_edge(tid + NT * i, k0);
-        }
-    };
-    auto store = [&](int sl, int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int idx = tid + NT * i;
-            if (!TA) {
-                const int row = idx / RQ, kq = (idx % RQ) * 4;
-                As[buf][kq + 0][row] = ra[sl][i].x;
-                As[buf][kq + 1][row] = ra[sl][i].y;
-                As[buf][kq + 2][row] = ra[sl][i].z;
-                As[buf][kq + 3][row] = ra[sl][i].w;
-            } else {
-                float *dst = &As[buf][idx >> 5][(idx & 31) * 4];
-                dst[0] = ra[sl][i].x;
-                dst[1] = ra[sl][i].y;
-                dst[2] = ra[sl][i].z;
-                dst[3] = ra[sl][i].w;
-            }
-            if (!TB) {
-                float *dst = &Bs[buf][idx >> 5][(idx & 31) * 4];
-                dst[0] = rb[sl][i].x;
-                dst[1] = rb[sl][i].y;
-                dst[2] = rb[sl][i].z;
-                dst[3] = rb[sl][i].w;
-            } else {
-                const int col = idx / RQ, kq = (idx % RQ) * 4;
-                Bs[buf][kq + 0][col] = rb[sl][i].x;
-                Bs[buf][kq + 1][col] = rb[sl][i].y;
-                Bs[buf][kq + 2][col] = rb[sl][i].z;
-                Bs[buf][kq + 3][col] = rb[sl][i].w;
-            }
-        }
-    };
-
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lr = lane & 31, lk = lane >> 5;
-
-    // One tile's MFMAs from LDS stage `buf`: all operand reads are issued
-    // first (for each k-pair kk the A value of the lane's row and the B
-    // values of its two column blocks); the MFMAs consume them in order as
-    // they land.
-    constexpr int cstep = CL == 0 ? 1 : CL == 1 ? 32 : 64;  // block 1's column offset
-    const int cbase = CL == 0 ? wn * 64 + 2 * lr : CL == 1 ? wn * 64 + lr : wn * 32 + lr;
-    auto compute = [&](int buf) __attribute__((always_inline)) {
-        const float *pa = &As[buf][lk][wm * 32 + lr];
-        const float *pb = &Bs[buf][lk][cbase];
-        float a[BK / 2];
-        float2 b[BK / 2];
-#pragma unroll
-        for (int kk = 0; kk < BK / 2; ++kk) {
-            a[kk] = pa[2 * kk * LdsA<TA>::S];
-            if constexpr (CL == 0)
-                b[kk] = *reinterpret_cast<const float2 *>(pb + 2 * kk * LdsB<TB>::S);
-            else
-                b[kk] = make_float2(pb[2 * kk * LdsB<TB>::S], pb[2 * kk * LdsB<TB>::S + cstep]);
-        }
-#pragma unroll
-        for (int kk = 0; kk < BK / 2; ++kk) {
-            acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[kk], b[kk].x, acc[0], 0, 0, 0);
-            acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[kk], b[kk].y, acc[1], 0, 0, 0);
-        }
-    };
-
-    // Pipeline: when iteration t starts, LDS stage t%2 holds tile t and
-    // register slot (t+j)%NS holds tile t+j for j = 1..NS (loads in flight;
-    // NS = SLOTS on interior tiles, 1 on edge tiles). Tile t+1 goes into the other stage
-    // (last read in iteration t-1, before its barrier), tile t+1+NS's global
-    // loads are issued into the slot that freed, and then the MFMAs of tile t
-    // run: a load has NS tiles of MFMAs to land, which covers HBM latency
-    // when the operands are in no cache (a layer's weights). One barrier per
-    // iteration. The loop is unrolled by the period of (stage, slot) so every
-    // slot index is a constant, and every step issues its loads
-    // unconditionally (tiles past the end reload the last one, which nothing
-    // reads): with the same loads on every path the compiler waits for
-    // exactly the oldest slot instead of draining all of them.
-    const int nk = (int)((kend - kbeg + BK - 1) / BK);
-    if (nk <= 0) return;
-    constexpr int U = NS % 2 == 0 ? NS : 2 * NS;
-    auto tile_k = [&](int t) __attribute__((always_inline)) {
-        return kbeg + (int64_t)min(t, nk - 1) * BK;
-    };
-    auto step = [&](auto uc, int it) __attribute__((always_inline)) {
-        constexpr int u = decltype(uc)::value;
-        store((u + 1) % NS, (u + 1) % 2);
-        load((u + 1) % NS, tile_k(it + 1 + NS));
-        compute(u % 2);
-        __syncthreads();
-    };
-    load(0, kbeg);
-    store(0, 0);
-    unroll_seq([&](auto jc) __attribute__((always_inline)) {
-        constexpr int j = decltype(jc)::value + 1;
-        load(j % NS, tile_k(j));
-    }, std::make_integer_sequence<int, NS>{});
-    __syncthreads();
-    int base = 0;
-    for (; base + U <= nk; base += U)
-        unroll_seq([&](auto uc) __attribute__((always_inline)) { step(uc, base + uc); },
-                   std::make_integer_sequence<int, U>{});
-    unroll_seq([&](auto uc) __attribute__((always_inline)) {
-        if (base + uc < nk) step(uc, base + uc);
-    }, std::make_integer_sequence<int, U>{});
-}
-
-// Tile t of the grouped order: GROUP_M tile rows at a time, column by column.
 // Split partials for the in-kernel reduction: stored through to memory and
 // read past the XCD-local L2 (device-scope relaxed atomics: sc1 stores and
 // loads), so the last split of a tile, on any XCD, reads every split's values.
@@ -528,339 +175,6 @@ __device__ __forceinline__ void split_reduce_tile(const KParams &p, int64_t m0, 
             for (int s = 1; s < p.splits; ++s) v = __fadd_rn(v, split_get(Q + (int64_t)s * total + u));
             float *dst = p.c + row * p.ldc + col + u;
             *dst = p.split_accum ? __fadd_rn(R[row * p.ldc + col + u], v) : v;
-        }
-    }
-}
-
-__device__ __forceinline__ void grouped_tile(const KParams &p, int t, int &tm, int &tn) {
-    const int per_group = GROUP_M * p.tiles_n;
-    const int group = t / per_group;
-    const int first_m = group * GROUP_M;
-    const int gsize = min(p.tiles_m - first_m, GROUP_M);
-    const int in_group = t - group * per_group;
-    tm = first_m + in_group % gsize;
-    tn = in_group / gsize;
-}
-
-template <bool TA, bool TB, int EPI, int CL = 0>
-__global__ __launch_bounds__(NT, 2) void gemm_f32_mfma(KParams p) {
-    static_assert(CL == 0 || EPI == EPI_STORE, "the RoPE column layouts store plain values");
-    __shared__ __attribute__((aligned(16))) float As[2][BK][LdsA<TA>::S];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BK][LdsB<TB>::S];
-
-    const int tid = threadIdx.x;
-
-    // XCD-aware renumbering of the whole tiles, then grouped tile order; the
-    // tail pieces (if any) follow the whole tiles.
-    int bid = blockIdx.x;
-    int piece = -1;
-    int64_t kbeg = (int64_t)blockIdx.z * p.k_per_split;
-    int64_t kend = min(p.k, kbeg + p.k_per_split);
-    if (p.tail_s > 1 && bid >= p.tail_first) {
-        piece = bid - p.tail_first;
-        bid = p.tail_first + piece / p.tail_s;
-        kbeg = (int64_t)(piece % p.tail_s) * p.tail_k;
-        kend = min(p.k, kbeg + p.tail_k);
-    } else {
-        const int nb = p.tail_s > 1 ? p.tail_first : (int)gridDim.x, q = nb >> 3, r = nb & 7;
-        const int xcd = bid & 7, local = bid >> 3;
-        bid = xcd * q + (xcd < r ? xcd : r) + local;
-    }
-    int tm, tn;
-    grouped_tile(p, bid, tm, tn);
-    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-
-    const int64_t batch = blockIdx.y;
-    const int split = blockIdx.z;
-    const float *__restrict__ A = p.a + batch * p.stride_a;
-    const float *__restrict__ B = p.b + batch * p.stride_b;
-    const int64_t M = p.m, N = p.n;
-
-    floatx16 acc[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[j][r] = p.acc_init;
-    // EPI_CE: the tile's target ids go to LDS before the K loop (whose
-    // barriers order them before the epilogue reads them)
-    __shared__ int ce_t[EPI == EPI_CE ? BM : 1];
-    if (EPI == EPI_CE && tid < BM) ce_t[tid] = m0 + tid < M ? p.ce_targets[m0 + tid] : -1;
-    const bool fast = p.vec_a && p.vec_b && m0 + BM <= M && n0 + BN <= N &&
-                      (kend - kbeg) % BK == 0;
-    if (fast)
-        gemm_mainloop<TA, TB, true, KSLOTS, CL, EPI == EPI_ACCUM>(p, A, B, m0, n0, kbeg, kend, As, Bs, acc);
-    else
-        gemm_mainloop<TA, TB, false, 1, CL>(p, A, B, m0, n0, kbeg, kend, As, Bs, acc);
-
-    // ---- epilogue: block j register r of lane l is C[row][col] with
-    // row = m0 + 32*wm + 8*(r/4) + 4*(l/32) + r%4 and, for CL 0,
-    // col = n0 + 64*wn + 2*(l%32) + j (the other layouts below).
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lr = lane & 31, lk = lane >> 5;
-    const int64_t col = n0 + wn * 64 + 2 * lr;
-    auto row_local = [&](int r) __attribute__((always_inline)) {
-        return wm * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
-    };
-    if (piece >= 0) {  // a tail piece: its partial tile, whole (edges included)
-        float *P = p.partial + (int64_t)piece * (BM * BN) + wn * 64 + 2 * lr;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            *reinterpret_cast<float2 *>(P + row_local(r) * BN) = make_float2(acc[0][r], acc[1][r]);
-        return;
-    }
-    if constexpr (CL != 0) {
-        // Column block j of lane lr is column c0 + j*half of C (half = 32 for
-        // CL 1, 64 for CL 2), c0 the lane's column in the first half of its
-        // head: RoPE (rope.rs:28-32) rotates the pair in registers, with the
-        // rope kernel's arithmetic, on the q and k heads (columns below
-        // rope_cols); the v heads are stored as they are.
-        constexpr int half = CL == 1 ? 32 : 64;
-        const int hc = CL == 1 ? lr : wn * 32 + lr;
-        const int64_t c0 = CL == 1 ? n0 + wn * 64 + lr : n0 + wn * 32 + lr;
-        const bool rot = p.rope_cos != nullptr && c0 < p.rope_cols;
-        float *C = p.c + batch * p.stride_c;
-        // The rows' table values are all read before the first store: the
-        // compiler cannot tell the tables from C, so a read placed after a
-        // store waits for that store's completion (one memory round trip per
-        // row). Rows past M read a valid table row (row % seq) and are dropped.
-        // Positions: the lane's first row modulo the sequence once; register
-        // r adds 8*(r/4) + r%4 < 28 to it, at most one wrap when seq >= 28.
-        float cs[16], sn[16];
-        if (rot) {
-            const uint32_t seq = (uint32_t)p.rope_seq;
-            const uint32_t base = (uint32_t)((m0 + row_local(0)) % p.rope_seq);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                uint32_t pos = base + (uint32_t)(8 * (r >> 2) + (r & 3));
-                if (seq < 28) pos %= seq;
-                else if (pos >= seq) pos -= seq;
-                const uint32_t t = pos * (uint32_t)half + (uint32_t)hc;
-                cs[r] = p.rope_cos[t];
-                sn[r] = p.rope_sin[t];
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t row = m0 + row_local(r);
-            if (row >= M) continue;
-            float x1 = acc[0][r], x2 = acc[1][r];
-            if (rot) {
-                const float y1 = x1 * cs[r] - x2 * sn[r];
-                const float y2 = x2 * cs[r] + x1 * sn[r];
-                x1 = y1;
-                x2 = y2;
-            }
-            if (c0 < N) C[row * p.ldc + c0] = x1;
-            if (c0 + half < N) C[row * p.ldc + c0 + half] = x2;
-        }
-        return;
-    }
-    if (p.splits > 1) {
-        // (summed by splitk_reduce: a tile's 2-16 partials are too much for
-        // one workgroup of the launch to add up at the end)
-        float *P = p.partial + (int64_t)split * M * N;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t row = m0 + row_local(r);
-            if (row < M) {
-                if (col < N) P[row * N + col] = acc[0][r];
-                if (col + 1 < N) P[row * N + col + 1] = acc[1][r];
-            }
-        }
-        return;
-    }
-    if constexpr (EPI == EPI_CE) {
-        // Cross-entropy partials of this tile's columns (ops_reduce.rs:236-259
-        // split by column tiles): per row, the max of the logits and the sum of
-        // exp(z - max) over the lane's two columns, over the 32 lanes of its
-        // half by DPP moves, then over the two waves sharing the rows through
-        // LDS. The lane holding a row's target column keeps its logit.
-        __shared__ float ce_m[2][BM], ce_s[2][BM];
-        constexpr float kLog2e = 1.4426950408889634f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int rl = row_local(r);
-            const int64_t row = m0 + rl;
-            const float v0 = acc[0][r], v1 = acc[1][r];
-            const float x0 = col < N ? v0 : -INFINITY, x1 = col + 1 < N ? v1 : -INFINITY;
-            const float mx = half_max32(fmaxf(x0, x1));
-            // exp(z - max) through the hardware's exp2 (no flush concern: the
-            // terms that matter are within a few hundred of 1)
-            const float e = half_sum32(
-                mx == -INFINITY ? 0.0f
-                                : __builtin_amdgcn_exp2f((x0 - mx) * kLog2e) +
-                                      __builtin_amdgcn_exp2f((x1 - mx) * kLog2e));
-            if (lr == 0) {
-                ce_m[wn][rl] = mx;
-                ce_s[wn][rl] = e;
-            }
-            const int t = ce_t[rl];
-            if (t == col) p.ce_zt[row] = v0;
-            if (t == col + 1) p.ce_zt[row] = v1;
-        }
-        __syncthreads();
-        if (tid < BM && m0 + tid < M) {
-            float m = ce_m[0][tid], sum = ce_s[0][tid];
-            lse_merge(m, sum, ce_m[1][tid], ce_s[1][tid]);
-            reinterpret_cast<float2 *>(p.ce_part)[(m0 + tid) * p.tiles_n + tn] =
-                make_float2(m, sum);
-        }
-        return;
-    }
-    float *C = p.c + batch * p.stride_c;
-    if (EPI == EPI_SWIGLU) {
-        // Packed columns interleave gate and up: column 2f is gate f, 2f+1 up f.
-        const int64_t f = col >> 1;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t row = m0 + row_local(r);
-            if (row >= M) continue;
-            if (p.aux && col + 1 < N)
-                *reinterpret_cast<float2 *>(p.aux + row * p.ldaux + col) =
-                    make_float2(acc[0][r], acc[1][r]);
-            if (f < p.swiglu_ff) C[row * p.ldc + f] = __fmul_rn(silu_fast(acc[0][r]), acc[1][r]);
-        }
-        return;
-    }
-    // The epilogues that read memory (the saved gate/up pairs, the residual)
-    // issue their reads ahead of their stores, 8 or 16 rows at a time: the
-    // destination may be the buffer read (in-place gradients, C += ...), so
-    // the compiler may not move a read past a store and would otherwise wait
-    // out one memory latency per row. Each lane reads only the elements it
-    // writes, so the early reads see the same values.
-    if (EPI == EPI_SWIGLU_BWD) {
-        // acc is dh[row][col, col+1]; their (g, u) pairs sit at aux columns
-        // 2*col .. 2*col+3 and the (dg, du) pairs go to the same columns of C.
-        if (m0 + BM <= M && n0 + BN <= N && p.ldc < (int64_t(1) << 20) &&
-            p.ldaux < (int64_t(1) << 20)) {
-            // The whole tile in range: unconditional buffer accesses from the
-            // tile's first row (see the residual epilogue below), eight rows'
-            // pairs read before their eight stores.
-            const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float *>(p.aux + m0 * p.ldaux), (short)0, kBufferRange, kBufferFlags);
-            const __amdgpu_buffer_rsrc_t rc =
-                __builtin_amdgcn_make_buffer_rsrc(C + m0 * p.ldc, (short)0, kBufferRange, kBufferFlags);
-            const uint32_t la = 4u * (uint32_t)p.ldaux, lc = 4u * (uint32_t)p.ldc;
-            const uint32_t va = (uint32_t)row_local(0) * la + 8u * (uint32_t)col;
-            const uint32_t vc = (uint32_t)row_local(0) * lc + 8u * (uint32_t)col;
-#pragma unroll
-            for (int r0 = 0; r0 < 16; r0 += 8) {
-                float4 g[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int r = r0 + j;
-                    g[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                          ra, va + (8 * (r >> 2) + (r & 3)) * la, 0, 0));
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int r = r0 + j;
-                    const float2 a = swiglu_bwd_f(acc[0][r], g[j].x, g[j].y);
-                    const float2 b2 = swiglu_bwd_f(acc[1][r], g[j].z, g[j].w);
-                    __builtin_amdgcn_raw_buffer_store_b128(
-                        __builtin_bit_cast(u32x4_t, make_float4(a.x, a.y, b2.x, b2.y)), rc,
-                        vc + (8 * (r >> 2) + (r & 3)) * lc, 0, 0);
-                }
-            }
-            return;
-        }
-#pragma unroll
-        for (int r0 = 0; r0 < 16; r0 += 8) {
-            float4 g[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int64_t row = m0 + row_local(r0 + j);
-                g[j] = row < M && col + 1 < N
-                           ? *reinterpret_cast<const float4 *>(p.aux + row * p.ldaux + 2 * col)
-                           : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int r = r0 + j;
-                const int64_t row = m0 + row_local(r);
-                if (row >= M) continue;
-                float *dst = C + row * p.ldc + 2 * col;
-                if (col + 1 < N) {
-                    const float2 a = swiglu_bwd_f(acc[0][r], g[j].x, g[j].y);
-                    const float2 b2 = swiglu_bwd_f(acc[1][r], g[j].z, g[j].w);
-                    *reinterpret_cast<float4 *>(dst) = make_float4(a.x, a.y, b2.x, b2.y);
-                } else if (col < N) {
-                    const float *gu = p.aux + row * p.ldaux + 2 * col;
-                    const float2 a = swiglu_bwd_f(acc[0][r], gu[0], gu[1]);
-                    dst[0] = a.x;
-                    dst[1] = a.y;
-                }
-            }
-        }
-        return;
-    }
-    const float *R = p.resid ? p.resid + batch * p.stride_c : C;
-    const bool pair = p.vec_c && col + 1 < N;
-    if (EPI == EPI_ACCUM && pair) {
-        float2 o[16];
-        if (m0 + BM <= M && p.ldc < (int64_t(1) << 21)) {
-            // Every row in range: no per-row branches, so the compiler counts
-            // the reads exactly and each store waits only for its own read
-            // (with the reads and stores under row tests, every store waited
-            // for all earlier stores as well: one store round trip per row).
-            // Buffer accesses from the tile's first row with 32-bit offsets
-            // (64-bit addresses for 16 rows took the kernel past the registers
-            // of four waves per SIMD). Each row's offset is added into the
-            // lane offset, never passed as the scalar offset: with computed
-            // scalar offsets the compiler reused an SGPR that a v_div_scale
-            // had just written as its carry-out, and one row of a tile read
-            // another row's values (found by the tail-pieces training test).
-            const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float *>(R + m0 * p.ldc), (short)0, kBufferRange, kBufferFlags);
-            const __amdgpu_buffer_rsrc_t rc =
-                __builtin_amdgcn_make_buffer_rsrc(C + m0 * p.ldc, (short)0, kBufferRange, kBufferFlags);
-            const uint32_t ldb4 = 4u * (uint32_t)p.ldc;
-            const uint32_t vo = (uint32_t)row_local(0) * ldb4 + 4u * (uint32_t)col;
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                o[r] = __builtin_bit_cast(
-                    float2, __builtin_amdgcn_raw_buffer_load_b64(rr, vo + (8 * (r >> 2) + (r & 3)) * ldb4, 0, 0));
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                __builtin_amdgcn_raw_buffer_store_b64(
-                    __builtin_bit_cast(u32x2_t, make_float2(__fadd_rn(o[r].x, acc[0][r]),
-                                                            __fadd_rn(o[r].y, acc[1][r]))),
-                    rc, vo + (8 * (r >> 2) + (r & 3)) * ldb4, 0, 0);
-            return;
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t row = m0 + row_local(r);
-            o[r] = row < M ? *reinterpret_cast<const float2 *>(R + row * p.ldc + col)
-                           : make_float2(0.f, 0.f);
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t row = m0 + row_local(r);
-            if (row >= M) continue;
-            *reinterpret_cast<float2 *>(C + row * p.ldc + col) =
-                make_float2(__fadd_rn(o[r].x, acc[0][r]), __fadd_rn(o[r].y, acc[1][r]));
-        }
-        return;
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int64_t row = m0 + row_local(r);
-        if (row >= M) continue;
-        float *dst = C + row * p.ldc + col;
-        const float *src = R + row * p.ldc + col;
-        float v0 = acc[0][r], v1 = acc[1][r];
-        if (pair) {
-            if (EPI == EPI_ACCUM) {
-                const float2 o = *reinterpret_cast<const float2 *>(src);
-                v0 = __fadd_rn(o.x, v0);
-                v1 = __fadd_rn(o.y, v1);
-            }
-            *reinterpret_cast<float2 *>(dst) = make_float2(v0, v1);
-        } else {
-            if (col < N) dst[0] = EPI == EPI_ACCUM ? __fadd_rn(src[0], v0) : v0;
-            if (col + 1 < N) dst[1] = EPI == EPI_ACCUM ? __fadd_rn(src[1], v1) : v1;
         }
     }
 }
@@ -1199,7 +513,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_small(KParams p) {
     // store, with no per-row branches (under row tests each read waited for
     // the stores before it: one memory round trip per row). Buffer accesses
     // from the tile's first row, each row's offset in the lane offset (as in
-    // the 128x128 kernel's epilogues).
+    // the large tiles' epilogues).
     const bool inside = m0 + SBM <= M && n0 + SBN <= N && p.ldc < (int64_t(1) << 21) &&
                         (EPI != EPI_SWIGLU_BWD || p.ldaux < (int64_t(1) << 21));
     const uint32_t lc = 4u * (uint32_t)p.ldc;
@@ -1523,172 +837,24 @@ __global__ __launch_bounds__(512) void mfma_peak_kernel(float *out, int n, uint3
     out[(int64_t)blockIdx.x * blockDim.x + threadIdx.x] = s;
 }
 
-// Sums the 128x128 kernel's split partials in split order, then applies the
-// epilogue. VEC: four consecutive columns per thread (n, ldc multiples of 4,
-// 16-byte aligned C, residual and partials), four splits' loads in flight.
-template <int EPI, bool VEC>
-__global__ __launch_bounds__(256) void splitk_reduce(const float *__restrict__ partial,
-                                                     float *c, const float *resid, int64_t m,
-                                                     int64_t n, int64_t ldc, int splits) {
-    const int64_t total = m * n;
-    if (VEC) {
-        for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; 4 * q < total;
-             q += (int64_t)gridDim.x * blockDim.x) {
-            const int64_t idx = 4 * q;
-            float4 acc = *reinterpret_cast<const float4 *>(partial + idx);
-            for (int s0 = 1; s0 < splits; s0 += 4) {
-                float4 v[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (s0 + u < splits)
-                        v[u] = *reinterpret_cast<const float4 *>(partial + (int64_t)(s0 + u) * total + idx);
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (s0 + u < splits) {
-                        acc.x = __fadd_rn(acc.x, v[u].x);
-                        acc.y = __fadd_rn(acc.y, v[u].y);
-                        acc.z = __fadd_rn(acc.z, v[u].z);
-                        acc.w = __fadd_rn(acc.w, v[u].w);
-                    }
-            }
-            const int64_t row = idx / n, col = idx - row * n;
-            float4 *dst = reinterpret_cast<float4 *>(c + row * ldc + col);
-            if (EPI == EPI_ACCUM) {
-                const float4 r = *reinterpret_cast<const float4 *>((resid ? resid : c) + row * ldc + col);
-                acc.x = __fadd_rn(r.x, acc.x);
-                acc.y = __fadd_rn(r.y, acc.y);
-                acc.z = __fadd_rn(r.z, acc.z);
-                acc.w = __fadd_rn(r.w, acc.w);
-            }
-            *dst = acc;
-        }
-        return;
-    }
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-         idx += (int64_t)gridDim.x * blockDim.x) {
-        float acc = partial[idx];
-        for (int s = 1; s < splits; ++s) acc = __fadd_rn(acc, partial[(int64_t)s * total + idx]);
-        const int64_t row = idx / n, col = idx - row * n;
-        float *dst = c + row * ldc + col;
-        if (EPI == EPI_ACCUM)
-            *dst = __fadd_rn((resid ? resid : c)[row * ldc + col], acc);
-        else
-            *dst = acc;
-    }
-}
-
-// The tail tiles of a balanced 128x128 launch: each element sums its tile's
-// tail_s pieces in piece order, then takes the epilogue (store, accumulate, or
-// the SwiGLU backward into the (dg, du) pairs). TAIL_PARTS workgroups per
-// tile (grid y), each thread four consecutive columns at a time with every
-// piece's load issued before the adds. VEC: 16-byte aligned C (and residual /
-// gate-up pairs) with ldc (ldaux) a multiple of 4, so interior columns move as
-// float4; otherwise, and past the matrix's last column, one at a time.
-constexpr int TAIL_PARTS = 8;
-
-template <int EPI, bool VEC>
-__global__ __launch_bounds__(256) void tail_reduce(KParams p) {
-    const int t = p.tail_first + (int)blockIdx.x;
-    int tm, tn;
-    grouped_tile(p, t, tm, tn);
-    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-    const float *part = p.partial + (int64_t)blockIdx.x * p.tail_s * (BM * BN);
-    const float *R = p.resid ? p.resid : p.c;
-    constexpr int PER = BM * BN / TAIL_PARTS;
-    for (int e = (int)blockIdx.y * PER + 4 * (int)threadIdx.x; e < ((int)blockIdx.y + 1) * PER;
-         e += 4 * 256) {
-        const int64_t row = m0 + e / BN, col = n0 + e % BN;
-        if (row >= p.m || col >= p.n) continue;
-        float4 v = *reinterpret_cast<const float4 *>(part + e);
-        for (int i0 = 1; i0 < p.tail_s; i0 += 4) {
-            float4 w[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (i0 + u < p.tail_s)
-                    w[u] = *reinterpret_cast<const float4 *>(part + (int64_t)(i0 + u) * (BM * BN) + e);
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (i0 + u < p.tail_s) {
-                    v.x = __fadd_rn(v.x, w[u].x);
-                    v.y = __fadd_rn(v.y, w[u].y);
-                    v.z = __fadd_rn(v.z, w[u].z);
-                    v.w = __fadd_rn(v.w, w[u].w);
-                }
-        }
-        const float vv[4] = {v.x, v.y, v.z, v.w};
-        if (VEC && col + 3 < p.n) {
-            if (EPI == EPI_SWIGLU_BWD) {
-                const float *gu = p.aux + row * p.ldaux + 2 * col;
-                const float4 a = *reinterpret_cast<const float4 *>(gu);
-                const float4 b = *reinterpret_cast<const float4 *>(gu + 4);
-                const float2 o0 = swiglu_bwd_f(vv[0], a.x, a.y), o1 = swiglu_bwd_f(vv[1], a.z, a.w);
-                const float2 o2 = swiglu_bwd_f(vv[2], b.x, b.y), o3 = swiglu_bwd_f(vv[3], b.z, b.w);
-                float4 *dst = reinterpret_cast<float4 *>(p.c + row * p.ldc + 2 * col);
-                dst[0] = make_float4(o0.x, o0.y, o1.x, o1.y);
-                dst[1] = make_float4(o2.x, o2.y, o3.x, o3.y);
-            } else if (EPI == EPI_ACCUM) {
-                const float4 r = *reinterpret_cast<const float4 *>(R + row * p.ldc + col);
-                *reinterpret_cast<float4 *>(p.c + row * p.ldc + col) =
-                    make_float4(__fadd_rn(r.x, vv[0]), __fadd_rn(r.y, vv[1]),
-                                __fadd_rn(r.z, vv[2]), __fadd_rn(r.w, vv[3]));
-            } else {
-                *reinterpret_cast<float4 *>(p.c + row * p.ldc + col) = v;
-            }
-            continue;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int64_t cu = col + u;
-            if (cu >= p.n) break;
-            if (EPI == EPI_SWIGLU_BWD) {
-                const float *gu = p.aux + row * p.ldaux + 2 * cu;
-                const float2 o = swiglu_bwd_f(vv[u], gu[0], gu[1]);
-                float *dst = p.c + row * p.ldc + 2 * cu;
-                dst[0] = o.x;
-                dst[1] = o.y;
-            } else if (EPI == EPI_ACCUM) {
-                p.c[row * p.ldc + cu] = __fadd_rn(R[row * p.ldc + cu], vv[u]);
-            } else {
-                p.c[row * p.ldc + cu] = vv[u];
-            }
-        }
-    }
-}
-
 template <bool TA, bool TB, int EPI>
-void launch(Context &ctx, const KParams &p, dim3 grid, bool small) {
+void launch(Context &ctx, const KParams &p, dim3 grid) {
     if constexpr (!TA && !TB && (EPI == EPI_STORE || EPI == EPI_SWIGLU)) {
-        if (small && p.norm_w) {
+        if (p.norm_w) {
             hipLaunchKernelGGL((gemm_f32_mfma_small<false, false, EPI, true>), grid, dim3(256), 0,
                                ctx.stream, p);
             return;
         }
     }
-    if constexpr (!TA && !TB && EPI == EPI_STORE) {
-        // RoPE in the 128x128 kernel's epilogue (heads of 64 or 128 columns)
-        if (!small && p.rope_cos) {
-            if (p.rope_hd == 64)
-                hipLaunchKernelGGL((gemm_f32_mfma<TA, TB, EPI, 1>), grid, dim3(NT), 0,
-                                   ctx.stream, p);
-            else
-                hipLaunchKernelGGL((gemm_f32_mfma<TA, TB, EPI, 2>), grid, dim3(NT), 0,
-                                   ctx.stream, p);
-            return;
-        }
-    }
-    if (small)
-        hipLaunchKernelGGL((gemm_f32_mfma_small<TA, TB, EPI, false>), grid, dim3(256), 0,
-                           ctx.stream, p);
-    else
-        hipLaunchKernelGGL((gemm_f32_mfma<TA, TB, EPI>), grid, dim3(NT), 0, ctx.stream, p);
+    hipLaunchKernelGGL((gemm_f32_mfma_small<TA, TB, EPI, false>), grid, dim3(256), 0,
+                       ctx.stream, p);
 }
 
 template <int EPI>
-void dispatch_t(Context &ctx, bool ta, bool tb, const KParams &p, dim3 grid, bool small) {
-    if (!ta && !tb) launch<false, false, EPI>(ctx, p, grid, small);
-    else if (!ta && tb) launch<false, true, EPI>(ctx, p, grid, small);
-    else if (ta && !tb) launch<true, false, EPI>(ctx, p, grid, small);
-    else launch<true, true, EPI>(ctx, p, grid, small);
+void dispatch_t(Context &ctx, bool ta, bool tb, const KParams &p, dim3 grid) {
+    if (!ta && !tb) launch<false, false, EPI>(ctx, p, grid);
+    else if (!ta) launch<false, true, EPI>(ctx, p, grid);
+    else launch<true, false, EPI>(ctx, p, grid);
 }
 
 bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
@@ -1699,15 +865,16 @@ namespace {
 
 int cus_of(const Context &ctx) { return ctx.cu_count > 0 ? ctx.cu_count : 256; }
 
-// Small tiles when the big ones cannot fill the chip and K is short enough
-// that one workgroup walking it alone stays cheap.
+// The fp32 MFMA tiles of 64x64: below one 128x128 tile per CU, for products of
+// at most 2^28 multiply-adds (above that the split tiles win: 2048 x 512 x 1024
+// 27.0 -> 20.9 us, 256 x 2048 x 1024 21.2 -> 18.6; at 2^28 the two meet, 4096 x
+// 512 x 128 10.3 against 13.7 us, 2048 x 128 x 1024 12.9 against 10.0), and
+// for the ones that take a norm in with their loads (K <= 256), whose own
+// launch costs more than the tiles gain.
 bool use_small(const Context &ctx, const GemmDesc &d) {
     const int64_t big_tiles = ((d.m + BM - 1) / BM) * ((d.n + BN - 1) / BN) * d.batch;
-    // (K up to 2048 for products of at most 2^29 multiply-adds: the 64x64
-    // tiles' splits sum in one launch, where the 128x128 splits need the
-    // reduce kernel; larger products keep the 128x128 tiles' operand reuse)
-    return d.force_splits == 0 && big_tiles < cus_of(ctx) &&
-           (d.k <= 1024 || (d.k <= 2048 && d.m * d.n * d.k <= (int64_t(1) << 29)));
+    if (big_tiles >= cus_of(ctx)) return false;
+    return (d.norm_w && d.k <= 256) || d.m * d.n * d.k <= (int64_t(1) << 28) / d.batch;
 }
 
 // When the K-split kernel runs: 1 for the small nn shapes of one matrix whose
@@ -1724,11 +891,11 @@ int ksplit_kind(const Context &ctx, const GemmDesc &d) {
     const int cus = cus_of(ctx);
     const bool plain = d.epi == EPI_STORE || d.epi == EPI_ACCUM;
     const int64_t small_tiles = ((d.m + SBM - 1) / SBM) * ((d.n + SBN - 1) / SBN);
+    const int64_t big_tiles = ((d.m + BM - 1) / BM) * ((d.n + BN - 1) / BN);
     if (use_small(ctx, d) && !d.ta && !d.tb && d.batch == 1 && d.k <= 480 &&
         small_tiles < 2 * cus && (plain || d.epi == EPI_SWIGLU))
         return 1;
-    const int64_t big_tiles = ((d.m + BM - 1) / BM) * ((d.n + BN - 1) / BN);
-    if (d.batch == 1 && d.force_splits == 0 && !(d.ta && d.tb) && plain && !d.norm_w &&
+    if (d.batch == 1 && plain && !d.norm_w &&
         !d.rope_cos && big_tiles < cus && d.m * d.n * d.k <= (int64_t(1) << 28))
         return 2;
     return 0;
@@ -1753,10 +920,9 @@ GemmFusion gemm_fusion(const Context &ctx, const GemmDesc &d) {
         f.rope = d.batch == 1 && d.epi == EPI_STORE && d.rope_hd > 0 && d.rope_hd <= 32 &&
                  32 % d.rope_hd == 0;
     } else {
-        // the 128x128 kernel rotates heads of 64 or 128 columns in registers;
-        // the norm stays a kernel of its own (in this kernel's loads it costs
-        // the registers of a ring slot, and the GEMM loses more than the norm
-        // kernel takes)
+        // the large tiles rotate heads of 64 or 128 columns in registers; the
+        // norm stays a kernel of its own (in their loads it would be redone by
+        // every column of tiles)
         f.rope = !d.ta && !d.tb && d.batch == 1 && d.epi == EPI_STORE &&
                  (d.rope_hd == 64 || d.rope_hd == 128);
     }
@@ -1764,15 +930,122 @@ GemmFusion gemm_fusion(const Context &ctx, const GemmDesc &d) {
 }
 
 int64_t gemm_ce_tiles(const Context &ctx, const GemmDesc &d) {
-    if (use_small(ctx, d) || d.batch != 1 || d.force_splits || d.ta || d.norm_w || d.rope_cos)
+    if (use_small(ctx, d) || d.batch != 1 || d.ta || d.norm_w || d.rope_cos)
         return 0;
     return (d.n + BN - 1) / BN;
 }
 
+namespace {
+
+struct TilePlan {
+    int tile = TILE_128, splits = 1;
+};
+
+// Split partials of the large tiles stay below this: the no-alloc entry point's
+// array holds them too, so both entry points take the same plan.
+constexpr int64_t kSplitBytes = kNoallocScratchBytes;
+
+// The tile and the K splits that an estimate of the launch makes shortest: with
+// G workgroups and q = ceil(G / CUs) on the busiest CU, 16 of K take
+// max(q * alone, G / CUs * full) us (kGemmTiles: a lone workgroup is bound by
+// its own steps, a full chip by its power), a tile's first loads and epilogue
+// about 6 steps more, and split sums a launch and the partials written and
+// read at 4.5 TB/s. Measured constants,
+// f32 TFLOP/s in brackets: 256x256 from 4096 x 2048 x 4096 on (220-228 against
+// 204-206 for 256x128), 256x128 for the grids of 100 to 500 of them (4096 x
+// 2048 x 2048: 197-202; 256x256 150, 128x128 174), 128x128 around one tile per
+// CU (1000 x 768 x 3072: 36.9 us against 40.9 and 41.8 for its neighbours),
+// 128x64 and 64x64 below (2048 x 512 x 1024 20.9 us against 32 for 128x128);
+// 1024 x 2048 x 4096 takes two splits of 256x128 (102 us against 117 whole).
+TilePlan choose_tile(const Context &ctx, const KParams &p, int64_t batch, int epi) {
+    const bool may_split = batch == 1 && (epi == EPI_STORE || epi == EPI_ACCUM) && !p.rope_cos;
+    const double cus = cus_of(ctx), ksteps = (double)((p.k + BK - 1) / BK);
+    TilePlan best;
+    double best_us = 0.0;
+    for (int tile = 0; tile < TILE_COUNT; ++tile) {
+        if (!gemm_tile_takes(p, epi, tile)) continue;
+        const GemmTileInfo &t = kGemmTiles[tile];
+        const double tiles = (double)((p.m + t.rows - 1) / t.rows) *
+                             (double)((p.n + t.cols - 1) / t.cols) * (double)batch;
+        for (int s = 1; s <= 8; s *= 2) {
+            // a split keeps 128 of K, as many as its prologue costs
+            if (s > 1 && (!may_split || p.k < 128 * s || s * p.m * p.n * 4 > kSplitBytes)) break;
+            const double g = tiles * s;
+            double us = std::max(std::ceil(g / cus) * t.alone, g / cus * t.full) * (ksteps / s + 6.0);
+            if (s > 1) us += 4.0 + (double)(s + 1) * (double)(p.m * p.n) * 4.0 / 4.5e6;
+            if (best_us == 0.0 || us < best_us) {
+                best_us = us;
+                best.tile = tile;
+                best.splits = s;
+            }
+        }
+    }
+    return best;
+}
+
+// mmh_gemm_noalloc's contract: which products it takes is stated in terms of a
+// plan of 128x128 tiles (the split that gives every CU a tile, or the last
+// tiles cut along K where they leave CUs idle) and its partials, and a product
+// that this plan cannot hold in 16 MiB is refused, whatever the kernels need.
+void check_noalloc(const Context &ctx, const GemmDesc &d) {
+    const int64_t cus = cus_of(ctx), limit = kNoallocLimitBytes;
+    const int64_t big = ((d.m + BM - 1) / BM) * ((d.n + BN - 1) / BN);
+    auto splits_of = [&](int64_t tiles, int64_t step) {
+        const int64_t steps = (d.k + step - 1) / step;
+        int64_t s = 1;
+        while (tiles * s < cus && s < 16 && steps / (s * 2) >= 8) s *= 2;
+        const int64_t per = (steps + s - 1) / s;
+        return (steps + per - 1) / per;
+    };
+    auto refuse_over = [&](int64_t splits) {
+        const int64_t need = splits * d.m * d.n * 4;
+        if (splits > 1 && need > limit)
+            fail(MMH_ERR_SHAPE, "gemm: the split-K partials of a " + std::to_string(d.m) + " x " +
+                                    std::to_string(d.n) + " product (" + std::to_string(splits) +
+                                    " splits) need " + std::to_string(need) +
+                                    " bytes; the scratch holds " + std::to_string(limit));
+        return splits > 1;
+    };
+    if (big < cus) {
+        // (partials of products this small, and of nn products with K up to
+        // 480, always fit: none, or at most K / 128 of them)
+        const int64_t mnk = d.m * d.n * d.k, tiles = ((d.m + 63) / 64) * ((d.n + 63) / 64);
+        if (mnk <= (int64_t(1) << 28)) return;
+        if (d.k <= 1024 || (d.k <= 2048 && mnk <= (int64_t(1) << 29))) {
+            if (d.ta || d.tb || d.k > 480 || tiles >= 2 * cus) refuse_over(splits_of(tiles, 32));
+            return;
+        }
+    }
+    const int64_t steps = (d.k + BK - 1) / BK;
+    if (refuse_over(splits_of(big, BK))) return;
+    const int64_t q = big / cus, r = big % cus;
+    if (q < 1 || r == 0) return;
+    int best_s = 1;
+    double best = (double)(q + 1);
+    for (int t : {2, 3, 4, 6, 8}) {
+        if (steps / t < 16) break;
+        const double span = (double)q + (double)((r * t + cus - 1) / cus) / t;
+        if (span < best - 1e-9) {
+            best = span;
+            best_s = t;
+        }
+    }
+    const int64_t need = r * best_s * BM * BN * 4;
+    if (best_s > 1 && best <= 0.95 * (double)(q + 1) && need > limit)
+        fail(MMH_ERR_SHAPE, "gemm: the tail pieces of a " + std::to_string(d.m) + " x " +
+                                std::to_string(d.n) + " product (" + std::to_string(r) +
+                                " tiles x " + std::to_string(best_s) + " pieces) need " +
+                                std::to_string(need) + " bytes; the scratch holds " +
+                                std::to_string(limit));
+}
+
+}  // namespace
+
 void gemm(Context &ctx, const GemmDesc &d) {
     if (d.m <= 0 || d.n <= 0 || d.k <= 0 || d.batch <= 0) fail(MMH_ERR_SHAPE, "gemm: empty shape");
+    if (d.ta && d.tb) fail(MMH_ERR_ARGUMENT, "gemm: one operand at most is transposed");
     if (d.epi == EPI_CE && (gemm_ce_tiles(ctx, d) == 0 || !d.ce_targets || !d.ce_part || !d.ce_zt))
-        fail(MMH_ERR_ARGUMENT, "gemm: the loss folds only into the 128x128 kernel of one matrix");
+        fail(MMH_ERR_ARGUMENT, "gemm: the loss folds only into the large tiles of one matrix");
     KParams p{};
     p.a = d.a;
     p.b = d.b;
@@ -1793,6 +1066,7 @@ void gemm(Context &ctx, const GemmDesc &d) {
     p.ce_targets = d.ce_targets;
     p.ce_part = d.ce_part;
     p.ce_zt = d.ce_zt;
+    p.ce_tiles = (int)((d.n + BN - 1) / BN);
     if (d.accumulate_into_c && (d.epi != EPI_ACCUM || d.resid))
         fail(MMH_ERR_ARGUMENT, "gemm: accumulate_into_c takes EPI_ACCUM into C itself");
     p.acc_init = d.accumulate_into_c ? -0.0f : 0.0f;
@@ -1807,10 +1081,10 @@ void gemm(Context &ctx, const GemmDesc &d) {
     const bool small = use_small(ctx, d);
     const int kind = ksplit_kind(ctx, d);
     const bool ksplit = kind != 0;
+    const bool tiled = !small && !ksplit;
     const GemmFusion fuse = gemm_fusion(ctx, d);
-    p.tiles_m = (int)(ksplit ? (d.m + 31) / 32 : small ? (d.m + SBM - 1) / SBM : (d.m + BM - 1) / BM);
-    p.tiles_n = (int)(ksplit ? (d.n + 31) / 32 : small ? (d.n + SBN - 1) / SBN : (d.n + BN - 1) / BN);
-    // The interior path addresses a tile with byte offsets below 2^31 (128 rows of ld).
+    if (d.scratch) check_noalloc(ctx, d);
+    // The interior path addresses a tile with byte offsets below 2^31.
     const int64_t off_limit = int64_t(1) << 29;
     p.vec_a = vec_a_of(d, d.a, d.lda);
     p.vec_b = (d.ldb % 4 == 0) && (d.batch == 1 || d.stride_b % 4 == 0) && aligned16(d.b) &&
@@ -1820,7 +1094,7 @@ void gemm(Context &ctx, const GemmDesc &d) {
 
     // RMSNorm of A: in the small kernel's loads, or first as its own kernel.
     if (d.norm_w) {
-        if (d.ta || d.batch != 1 || d.force_splits > 0)
+        if (d.ta || d.batch != 1)
             fail(MMH_ERR_ARGUMENT, "gemm: the A-row norm takes one row-major A");
         if (fuse.norm) {
             p.norm_w = d.norm_w;
@@ -1834,36 +1108,49 @@ void gemm(Context &ctx, const GemmDesc &d) {
         }
     }
 
+    // RoPE in the small and large tiles' epilogues (gemm_fusion), where the K
+    // is not split.
+    const bool rope = d.rope_cos != nullptr;
+    if (rope) {
+        if (d.batch != 1 || d.rope_hd <= 0 || d.rope_hd % 2 || d.rope_seq <= 0 ||
+            d.m % d.rope_seq || d.rope_cols % d.rope_hd || d.rope_cols > d.n || !d.rope_sin ||
+            d.m > INT32_MAX || d.n > INT32_MAX)
+            fail(MMH_ERR_ARGUMENT, "gemm: bad rope arguments");
+        if (fuse.rope) {
+            p.rope_cos = d.rope_cos;
+            p.rope_sin = d.rope_sin;
+            p.rope_seq = (int)d.rope_seq;
+            p.rope_hd = (int)d.rope_hd;
+            p.rope_cols = (int)d.rope_cols;
+        }
+    }
+
+    TilePlan plan;
+    if (tiled) plan = choose_tile(ctx, p, d.batch, d.epi);
+    const int64_t tile_m = ksplit ? 32 : tiled ? kGemmTiles[plan.tile].rows : SBM;
+    const int64_t tile_n = ksplit ? 32 : tiled ? kGemmTiles[plan.tile].cols : SBN;
+    p.tiles_m = (int)((d.m + tile_m - 1) / tile_m);
+    p.tiles_n = (int)((d.n + tile_n - 1) / tile_n);
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-    const int64_t kstep = ksplit ? 32 : small ? SBK : BK;
+    const int64_t kstep = ksplit ? 32 : tiled ? BK : SBK;
     const int64_t ktiles = (d.k + kstep - 1) / kstep;
     int splits = 1;
-    if (d.force_splits > 0) {
-        splits = d.force_splits;
+    if (tiled) {
+        splits = plan.splits;
     } else if (kind == 2) {
         // Up to two workgroups per CU, each split keeping >= 4 steps of 32
         // (a step per wave at least).
         while (tiles * splits < 2 * (int64_t)cus && splits < 64 && ktiles / (splits * 2) >= 4)
             splits *= 2;
     } else if (!ksplit && d.batch == 1 && d.epi != EPI_SWIGLU && d.epi != EPI_SWIGLU_BWD) {
-        if (small) {
-            // Split only while a split keeps >= 8 steps of 32 (the reduce
-            // launch costs about what 8 steps do) and the grid is below a
-            // workgroup per CU.
-            while (tiles * splits < cus && splits < 16 && ktiles / (splits * 2) >= 8)
-                splits *= 2;
-        } else {
-            // Fill the chip: a tile per CU (two, with twice the split partials
-            // written and summed, measured 7-10% slower from 1 GFLOP up: the
-            // sweep's dB forms, the training's 2048 x 2048 weight gradient), at
-            // least 8 K-steps per split.
-            const int64_t target = (int64_t)cus;
-            while (tiles * splits < target && splits < 16 && ktiles / (splits * 2) >= 8)
-                splits *= 2;
-        }
+        // Split only while a split keeps >= 8 steps of 32 (the reduce
+        // launch costs about what 8 steps do) and the grid is below a
+        // workgroup per CU.
+        while (tiles * splits < cus && splits < 16 && ktiles / (splits * 2) >= 8)
+            splits *= 2;
     }
     if (d.batch > 1 || d.epi == EPI_SWIGLU || d.epi == EPI_SWIGLU_BWD || d.epi == EPI_CE ||
-        p.norm_w || kind == 1)
+        p.norm_w || p.rope_cos || kind == 1)
         splits = 1;
     const int64_t kt_per = (ktiles + splits - 1) / splits;
     p.k_per_split = kt_per * kstep;
@@ -1873,8 +1160,8 @@ void gemm(Context &ctx, const GemmDesc &d) {
         // 64x64 and 32x32 tiles: the last split of each tile sums the
         // partials in split order and applies the epilogue (one launch;
         // every such grid has fewer tiles than two per CU, far below the
-        // counters); 128x128 tiles: splitk_reduce after the launch
-        if (small || ksplit) {
+        // counters); the large tiles: splitk_reduce after the launch
+        if (!tiled) {
             p.tickets = d.scratch ? d.scratch_tickets : ctx.tickets;
             if (!p.tickets || tiles > Context::kTickets)
                 fail(MMH_ERR_OTHER, "gemm: no split counters for " + std::to_string(tiles) + " tiles");
@@ -1882,75 +1169,17 @@ void gemm(Context &ctx, const GemmDesc &d) {
         }
         const size_t need_bytes = (size_t)splits * d.m * d.n * 4;
         if (d.scratch) {
-            if (need_bytes > d.scratch_bytes)
-                fail(MMH_ERR_SHAPE, "gemm: the split-K partials of a " + std::to_string(d.m) +
-                                        " x " + std::to_string(d.n) + " product (" +
-                                        std::to_string(splits) + " splits) need " +
-                                        std::to_string(need_bytes) + " bytes; the scratch holds " +
-                                        std::to_string(d.scratch_bytes));
+            if (need_bytes > d.scratch_bytes)  // (check_noalloc and kSplitBytes rule it out)
+                fail(MMH_ERR_OTHER, "gemm: the split-K partials do not fit the scratch");
             p.partial = d.scratch;
         } else {
             p.partial = static_cast<float *>(ctx.get_scratch(need_bytes));
         }
     }
 
-    // RoPE in the small kernel's epilogue when a head fits 32 columns.
-    const bool rope = d.rope_cos != nullptr;
-    if (rope) {
-        if (d.batch != 1 || d.rope_hd <= 0 || d.rope_hd % 2 || d.rope_seq <= 0 ||
-            d.m % d.rope_seq || d.rope_cols % d.rope_hd || d.rope_cols > d.n || !d.rope_sin ||
-            d.m > INT32_MAX || d.n > INT32_MAX)
-            fail(MMH_ERR_ARGUMENT, "gemm: bad rope arguments");
-        if (fuse.rope && splits == 1) {
-            p.rope_cos = d.rope_cos;
-            p.rope_sin = d.rope_sin;
-            p.rope_seq = (int)d.rope_seq;
-            p.rope_hd = (int)d.rope_hd;
-            p.rope_cols = (int)d.rope_cols;
-        }
-    }
-
-    // Tail balance for the 128x128 kernel: with tiles = q * CUs + R (q >= 1,
-    // R > 0) the CUs that draw q + 1 tiles set the launch's length. The last R
-    // tiles instead split K into s pieces (each a workgroup of its own, at
-    // least 16 K-steps long), so every CU takes about q + R/CUs tiles' work;
-    // tail_reduce sums each tile's pieces in order. Chosen when it shortens
-    // the longest CU's share by at least 5%.
     const int epi = splits > 1 ? EPI_STORE : d.epi;
-    if (!ksplit && !small && splits == 1 && d.batch == 1 && !p.rope_cos && d.force_splits == 0 &&
-        (epi == EPI_STORE || epi == EPI_ACCUM || epi == EPI_SWIGLU_BWD)) {
-        const int64_t cus = cus_of(ctx), q = tiles / cus, R = tiles % cus;
-        int best_s = 1;
-        double best = (double)(q + (R > 0));
-        for (int s : {2, 3, 4, 6, 8}) {
-            if (q < 1 || R == 0 || ktiles / s < 16) break;
-            const double span = (double)q + (double)((R * s + cus - 1) / cus) / s;
-            if (span < best - 1e-9) {
-                best = span;
-                best_s = s;
-            }
-        }
-        const size_t need = (size_t)R * best_s * BM * BN * 4;
-        if (best_s > 1 && best <= 0.95 * (double)(q + 1)) {
-            // the choice never depends on the caller's scratch, so a fixed
-            // scratch gives the same summation order (and bits) as the
-            // workspace, or the call is refused
-            if (d.scratch && need > d.scratch_bytes)
-                fail(MMH_ERR_SHAPE, "gemm: the tail pieces of a " + std::to_string(d.m) + " x " +
-                                        std::to_string(d.n) + " product (" + std::to_string(R) +
-                                        " tiles x " + std::to_string(best_s) + " pieces) need " +
-                                        std::to_string(need) + " bytes; the scratch holds " +
-                                        std::to_string(d.scratch_bytes));
-            p.tail_first = (int)(tiles - R);
-            p.tail_s = best_s;
-            p.tail_k = (ktiles + best_s - 1) / best_s * BK;
-            p.partial = d.scratch ? d.scratch : static_cast<float *>(ctx.get_scratch(need));
-        }
-    }
-    const int64_t tail_pieces = p.tail_s > 1 ? (tiles - p.tail_first) * p.tail_s : 0;
-    const int64_t grid_x = p.tail_s > 1 ? p.tail_first + tail_pieces : tiles;
-    if (grid_x > 0x7fffffff || d.batch > 65535) fail(MMH_ERR_SHAPE, "gemm: grid too large");
-    dim3 grid((unsigned)grid_x, (unsigned)d.batch, (unsigned)splits);
+    if (tiles > 0x7fffffff || d.batch > 65535) fail(MMH_ERR_SHAPE, "gemm: grid too large");
+    dim3 grid((unsigned)tiles, (unsigned)d.batch, (unsigned)splits);
     if (ksplit) {
         // The k-contiguous operands (A when !ta, B when tb, the norm weights)
         // decide between vector and predicated reads (vec_a / vec_b hold
@@ -1969,62 +1198,21 @@ void gemm(Context &ctx, const GemmDesc &d) {
         else
             (epi == EPI_ACCUM ? launch_ksplit<true, false, EPI_ACCUM>
                               : launch_ksplit<true, false, EPI_STORE>)(ctx, p, grid, mode);
-    } else if (epi == EPI_CE) {
-        if (d.tb)
-            hipLaunchKernelGGL((gemm_f32_mfma<false, true, EPI_CE>), grid, dim3(NT), 0,
-                               ctx.stream, p);
-        else
-            hipLaunchKernelGGL((gemm_f32_mfma<false, false, EPI_CE>), grid, dim3(NT), 0,
-                               ctx.stream, p);
+    } else if (tiled) {
+        launch_gemm_tiles(ctx, p, grid, d.ta, d.tb, epi, plan.tile);
     } else if (epi == EPI_SWIGLU) {
         if (d.ta || d.tb) fail(MMH_ERR_ARGUMENT, "gemm: swiglu epilogue needs the nn form");
-        launch<false, false, EPI_SWIGLU>(ctx, p, grid, small);
+        launch<false, false, EPI_SWIGLU>(ctx, p, grid);
     } else if (epi == EPI_SWIGLU_BWD) {
         if (d.ta || !d.tb) fail(MMH_ERR_ARGUMENT, "gemm: swiglu backward epilogue needs the nt form");
-        launch<false, true, EPI_SWIGLU_BWD>(ctx, p, grid, small);
+        launch<false, true, EPI_SWIGLU_BWD>(ctx, p, grid);
     } else if (epi == EPI_ACCUM) {
-        dispatch_t<EPI_ACCUM>(ctx, d.ta, d.tb, p, grid, small);
+        dispatch_t<EPI_ACCUM>(ctx, d.ta, d.tb, p, grid);
     } else {
-        dispatch_t<EPI_STORE>(ctx, d.ta, d.tb, p, grid, small);
+        dispatch_t<EPI_STORE>(ctx, d.ta, d.tb, p, grid);
     }
     check_hip(hipGetLastError(), "gemm launch");
-    if (splits > 1 && !p.tickets) {
-        const int64_t total = d.m * d.n;
-        const bool vec = d.n % 4 == 0 && d.ldc % 4 == 0 && aligned16(d.c) &&
-                         aligned16(p.partial) && (!d.resid || aligned16(d.resid));
-        const int64_t items = vec ? total / 4 : total;
-        const unsigned blocks = (unsigned)std::min<int64_t>((items + 255) / 256, 8192);
-#define MMH_SPLITK(E, V)                                                                   \
-    hipLaunchKernelGGL((splitk_reduce<E, V>), dim3(blocks), dim3(256), 0, ctx.stream, p.partial, \
-                       d.c, E == EPI_ACCUM ? d.resid : nullptr, d.m, d.n, d.ldc, splits)
-        if (d.epi == EPI_ACCUM) {
-            if (vec) MMH_SPLITK(EPI_ACCUM, true); else MMH_SPLITK(EPI_ACCUM, false);
-        } else {
-            if (vec) MMH_SPLITK(EPI_STORE, true); else MMH_SPLITK(EPI_STORE, false);
-        }
-#undef MMH_SPLITK
-        check_hip(hipGetLastError(), "split-k reduce launch");
-    }
-    if (p.tail_s > 1) {
-        const dim3 rg((unsigned)(tiles - p.tail_first), TAIL_PARTS);
-        const bool vec = d.ldc % 4 == 0 && aligned16(d.c) && (!d.resid || aligned16(d.resid)) &&
-                         (epi != EPI_SWIGLU_BWD || (d.ldaux % 4 == 0 && aligned16(d.aux)));
-#define MMH_TAIL(E)                                                                        \
-    do {                                                                                   \
-        if (vec)                                                                           \
-            hipLaunchKernelGGL((tail_reduce<E, true>), rg, dim3(256), 0, ctx.stream, p);   \
-        else                                                                               \
-            hipLaunchKernelGGL((tail_reduce<E, false>), rg, dim3(256), 0, ctx.stream, p);  \
-    } while (0)
-        if (epi == EPI_SWIGLU_BWD)
-            MMH_TAIL(EPI_SWIGLU_BWD);
-        else if (epi == EPI_ACCUM)
-            MMH_TAIL(EPI_ACCUM);
-        else
-            MMH_TAIL(EPI_STORE);
-#undef MMH_TAIL
-        check_hip(hipGetLastError(), "tail reduce launch");
-    }
+    if (splits > 1 && !p.tickets) launch_splitk_reduce(ctx, p, d.epi);
     if (rope && !p.rope_cos)
         launch_rope_strided(ctx, d.c, d.rope_seq * d.ldc, d.rope_hd, d.ldc, d.m / d.rope_seq,
                             d.rope_cols / d.rope_hd, d.rope_seq, d.rope_hd, d.rope_cos,

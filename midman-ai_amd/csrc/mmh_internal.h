@@ -109,13 +109,18 @@ void release_models_of(mmh_handle ctx);
 // EPI_SWIGLU: columns (2f, 2f+1) are (gate f, up f); C[row][f] = silu(gate)*up,
 // and aux (when set) receives the raw pair. EPI_SWIGLU_BWD: acc is dh [M, ff];
 // with (g, u) = aux[row][2f, 2f+1], C[row][2f, 2f+1] = (dg, du) (C may be aux).
-// EPI_CE: C is not written; the products are logits, and each 128-column tile
+// EPI_CE: C is not written; the products are logits, and each 128 columns
 // tn of row i leaves ce_part[(i * tiles + tn) * 2 + {0, 1}] = (max, sum of
 // exp(z - max)) over its columns, and the tile holding column ce_targets[i]
 // leaves that logit in ce_zt[i] (the head GEMM with the loss folded in; see
 // gemm_ce_tiles and launch_ce_combine).
 enum Epilogue : int { EPI_STORE = 0, EPI_ACCUM = 1, EPI_SWIGLU = 2, EPI_SWIGLU_BWD = 3,
                       EPI_CE = 4 };
+
+// mmh_gemm_noalloc: the partials of the plan its contract is stated in, and the
+// array the kernels' own partials live in (their plans stay below it).
+constexpr int64_t kNoallocLimitBytes = int64_t(16) << 20;
+constexpr int64_t kNoallocScratchBytes = int64_t(64) << 20;
 
 struct GemmDesc {
     const float *a = nullptr;
@@ -130,7 +135,6 @@ struct GemmDesc {
     const float *resid = nullptr;  // EPI_ACCUM: residual source (ldc layout); null = C
     float *aux = nullptr;          // EPI_SWIGLU(_BWD): interleaved gate/up pairs
     int64_t ldaux = 0;
-    int force_splits = 0;   // 0 = heuristic
     // RMSNorm of A's rows first (norm.rs:21-39; nn form, batch 1): A is x and
     // the product uses (x * inv) * norm_w with inv = (mean(x^2) + eps)^-1/2.
     // Folded into the small-tile kernel's loads when K <= 256; otherwise the
@@ -144,13 +148,13 @@ struct GemmDesc {
     // otherwise by the rope kernel after the product. Same bits either way.
     const float *rope_cos = nullptr, *rope_sin = nullptr;
     int64_t rope_seq = 0, rope_hd = 0, rope_cols = 0;
-    // EPI_CE (batch 1, the 128x128 kernel only): targets [m] on the device,
+    // EPI_CE (batch 1, the large tiles only): targets [m] on the device,
     // partials [m, gemm_ce_tiles, 2] and target logits [m] out.
     const int32_t *ce_targets = nullptr;
     float *ce_part = nullptr, *ce_zt = nullptr;
     // Device memory for the split-K partials supplied by the caller (null: the
-    // context's growable workspace). gemm() fails with MMH_ERR_SHAPE when the
-    // partials of the split it chooses need more than scratch_bytes.
+    // context's growable workspace), kNoallocScratchBytes of it: gemm() then
+    // takes what mmh_gemm_noalloc takes and refuses the rest (MMH_ERR_SHAPE).
     float *scratch = nullptr;
     size_t scratch_bytes = 0;
     // With scratch: kTickets zeroed tile counters for the in-kernel split

@@ -3,10 +3,9 @@
 // harnesses that forbid hipMalloc). The only device memory the GEMM needs
 // beyond its operands is the split-K partials ([splits, m, n] f32, written in
 // full by the splits and summed in split order by the last split of each
-// tile) with one counter per tile, and the tail pieces of the 128x128 kernel
-// (summed by tail_reduce); here they live in file-scope device arrays of
-// fixed size instead of the context's growable workspace and counters, so no
-// call allocates or frees anything.
+// tile, or by a second kernel) with one counter per tile; here they live in
+// file-scope device arrays of fixed size instead of the context's growable
+// workspace and counters, so no call allocates or frees anything.
 //
 // The arrays exist once per GPU (each device that loads this code object
 // holds its own copy until the process ends). Their device addresses are
@@ -14,8 +13,8 @@
 // current, and only those addresses are ever handed to kernels. Every call on
 // one GPU shares them: calls that overlap on one GPU (two streams, two
 // contexts, two threads) race on them. Nothing in them needs clearing between
-// calls: each split or piece writes every element of its partial tile before
-// it is summed, and the counters start at zero (the arrays are zero when the
+// calls: each split writes every element of its partial tile before it is
+// summed, and the counters start at zero (the arrays are zero when the
 // code object loads) and are reset by the split that completes a tile.
 #include <mutex>
 
@@ -24,9 +23,7 @@
 namespace mmh {
 namespace {
 
-constexpr size_t kScratchBytes = size_t(16) << 20;  // 16 MiB per GPU: the benchmark sweep's largest partials
-
-static __device__ __align__(256) float scratch[kScratchBytes / 4];
+static __device__ __align__(256) float scratch[kNoallocScratchBytes / 4];
 // The split-K tile counters (zero when the code object loads; the last split
 // of a tile resets its counter, so they are zero between calls).
 static __device__ __align__(256) int32_t scratch_tickets[Context::kTickets];
@@ -91,7 +88,7 @@ int32_t mmh_gemm_noalloc(mmh_handle ctx, int32_t form, const float *a, const flo
         d.epi = accumulate ? EPI_ACCUM : EPI_STORE;
         d.accumulate_into_c = accumulate != 0;
         d.scratch = scratch_of(cx, &d.scratch_tickets);
-        d.scratch_bytes = kScratchBytes;
+        d.scratch_bytes = kNoallocScratchBytes;
         gemm(cx, d);
         return MMH_OK;
     });

@@ -1,0 +1,115 @@
+"""GPU checks of the split GEMM tiles (gemm_split.hip): f32 products from six
+bf16 MFMA products of exact three-way splits, against 64-bit sums.
+
+Bound per element: with S = sum_p |a_p b_p|, the three products left out are
+below 3 * 2^-24 S; the matrix core rounds the running sum once per product
+group of 16 k, six groups per 16 k, each below 2^-23 S (it may truncate); a K
+split adds at most 8 partials. So |err| <= (6 * ceil(k / 16) + 16) * 2^-23 * S.
+"""
+import numpy as np
+import pytest
+
+import midman_hip as mh
+
+pytestmark = pytest.mark.gpu
+
+# (m, k, n) with row, column and K remainders; which tile the choice in
+# gemm.hip gives each on 256 CUs
+SHAPES = [
+    ("256x256, K tail", 3900, 100, 4000),
+    ("256x128, whole steps", 2050, 64, 4100),
+    ("256x128 in 2 splits", 1000, 2050, 4100),
+    ("128x128, 2 wave groups, odd step and tail", 1000, 777, 3071),
+    ("128x128 in splits", 1003, 1517, 770),
+    ("128x64, an odd step", 2000, 528, 1001),
+    ("64x64, 4 wave groups, 3 odd steps and a tail", 1030, 569, 515),
+    ("64x64 in splits", 300, 5003, 301),
+    ("64x64, fewer whole steps than wave groups", 2300, 50, 2301),
+]
+
+
+def run(ctx, form, a, b, c0=None):
+    m, k, n = a.shape[0], a.shape[1], b.shape[1]
+    A = ctx.to_device(np.ascontiguousarray(a.T) if form == "tn" else a)
+    B = ctx.to_device(np.ascontiguousarray(b.T) if form == "nt" else b)
+    C = ctx.to_device(c0) if c0 is not None else ctx.empty((m, n))
+    mh.gemm(ctx, form, A, B, C, m, k, n, accumulate=c0 is not None)
+    out = C.numpy()
+    for x in (A, B, C):
+        x.free()
+    return out
+
+
+def check(out, a, b, c0=None):
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    k = a.shape[1]
+    bound = (6 * -(-k // 16) + 16) * 2.0**-23 * size + 2.0**-140
+    if c0 is not None:
+        want = want + c0
+        bound = bound + 2.0**-23 * (np.abs(c0) + size)
+    worst = float(np.max(np.abs(out - want) / bound))
+    print(f"  max err / bound {worst:.3g}", flush=True)
+    assert worst <= 1.0
+
+
+@pytest.mark.parametrize("what,m,k,n", SHAPES, ids=[s[0] for s in SHAPES])
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+def test_tile_edges(ctx, what, m, k, n, form):
+    print(f"\n[gemm split] {what}: {form} {m}x{k}x{n}", flush=True)
+    r = np.random.default_rng(m + k + n)
+    a = r.standard_normal((m, k), dtype=np.float32)
+    b = r.standard_normal((k, n), dtype=np.float32)
+    c0 = r.standard_normal((m, n), dtype=np.float32)
+    check(run(ctx, form, a, b), a, b)
+    check(run(ctx, form, a, b, c0), a, b, c0)
+
+
+@pytest.mark.parametrize("what,m,k,n", SHAPES, ids=[s[0] for s in SHAPES])
+@pytest.mark.parametrize("lo,hi", [(-60, 60), (-126, -90), (100, 126)])
+def test_every_exponent(ctx, what, m, k, n, lo, hi):
+    # magnitudes from 2^lo to 2^hi on one side and their reciprocals' range on
+    # the other: pieces that would be subnormal in bf16 (below 2^-102) and
+    # values above its largest finite one take the fp32 products
+    print(f"\n[gemm split] {what}: exponents {lo}..{hi}, {m}x{k}x{n}", flush=True)
+    r = np.random.default_rng(m * 3 + k + hi)
+    signs = lambda s: r.choice(np.float32([-1, 1]), s)  # noqa: E731
+    mant = lambda s: r.uniform(1, 2, s).astype(np.float32)  # noqa: E731
+    a = signs((m, k)) * np.ldexp(mant((m, k)), r.integers(lo, hi + 1, (m, k))).astype(np.float32)
+    span = (-hi, -lo) if lo > -100 and hi < 100 else ((0, 20) if hi < 0 else (-40, -20))
+    b = signs((k, n)) * np.ldexp(mant((k, n)), r.integers(span[0], span[1] + 1, (k, n))).astype(np.float32)
+    check(run(ctx, "nn", a, b), a, b)
+
+
+@pytest.mark.parametrize("what,m,k,n", SHAPES, ids=[s[0] for s in SHAPES])
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+def test_special_values(ctx, what, m, k, n, form):
+    # inf, NaN, the largest float, subnormals and -0 in single rows, columns
+    # and the last k of integer operands: exact sums, so the bits are the
+    # scalar rules' (float64 arithmetic rounded once)
+    print(f"\n[gemm split] special values, {what}: {form} {m}x{k}x{n}", flush=True)
+    r = np.random.default_rng(k)
+    a = r.integers(-3, 4, (m, k)).astype(np.float32)
+    b = r.integers(-3, 4, (k, n)).astype(np.float32)
+    a[1, k - 1], a[m - 1, 0] = np.inf, np.nan
+    b[k - 1, n - 1] = -np.inf
+    big = np.finfo(np.float32).max
+    a[m // 2], b[:, n // 2] = 0.0, 0.0
+    a[m // 2, 0], b[0, n // 2] = big, 1.0
+    tiny = np.float32(2.0**-149)
+    a[m // 3] = 0.0
+    a[m // 3, k // 2] = 3 * tiny
+    a[m // 4] = -0.0
+    c0 = np.zeros((m, n), np.float32)
+    c0[m // 4] = -0.0
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    out = run(ctx, form, a, b)
+    assert np.array_equal(out, want, equal_nan=True)
+    fin = np.isfinite(want)
+    acc = run(ctx, form, a, b, c0)
+    assert np.array_equal(acc[fin], (want + c0)[fin])
+    # a row of -0 times positives keeps C's -0
+    b2 = np.abs(np.where(np.isfinite(b), b, 1)).astype(np.float32) + 1
+    acc = run(ctx, form, a, b2, c0)
+    assert np.all(np.signbit(acc[m // 4])) and np.all(acc[m // 4] == 0.0)
