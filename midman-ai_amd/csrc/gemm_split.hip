@@ -60,14 +60,12 @@
 // tiles, walked in groups of tile rows so that the tiles an XCD holds at once
 // share A rows and B columns in its L2.
 #include "mmh_gemm.h"
+#include "mmh_split.h"
 
 #include <algorithm>
-#include <utility>
 
 namespace mmh {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // Reductions over each 32-lane half of a wave with DPP moves (quad permutes,
 // then rotations within a 16-lane row) and one v_permlane16_swap across the
@@ -114,44 +112,6 @@ __device__ __forceinline__ void grouped_tile(const KParams &p, int group, int t,
     tn = in_group / gsize;
 }
 constexpr int group_rows(int tile_m) { return 1024 / tile_m; }
-
-// Calls f(integral_constant<int, i>) for i = 0..n-1, so that i is a
-// compile-time constant in each call (register-slot indices stay static).
-template <class F, int... Is>
-__device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, Is...>) {
-    (f(std::integral_constant<int, Is>{}), ...);
-}
-
-// Below this (2 * bits - 1 of 2^-102) a non-zero value's pieces may be
-// subnormal in bf16.
-constexpr uint32_t kTiny = 0x18ffffffu;
-
-// (bf16(x), bf16(y)), rounded to nearest even. As assembly because from the
-// cast the compiler converts x a second time on its own for the remainder.
-__device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
-    uint32_t r;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
-    return r;
-}
-
-// E values of consecutive k as three pieces of E bf16 each; tiny follows the
-// smallest 2 * |bits| - 1 (zeros wrap to the largest).
-template <int E>
-__device__ __forceinline__ void split_values(const float (&v)[E], uint32_t (&o)[3][E / 2],
-                                             uint32_t &tiny) {
-#pragma unroll
-    for (int i = 0; i < E / 2; ++i) {
-        const float x = v[2 * i], y = v[2 * i + 1];
-        const uint32_t h = pack_bf16(x, y);
-        const float rx = x - __uint_as_float(h << 16), ry = y - __uint_as_float(h & 0xffff0000u);
-        const uint32_t m = pack_bf16(rx, ry);
-        const float sx = rx - __uint_as_float(m << 16), sy = ry - __uint_as_float(m & 0xffff0000u);
-        o[0][i] = h;
-        o[1][i] = m;
-        o[2][i] = pack_bf16(sx, sy);
-        tiny = min(tiny, min((__float_as_uint(x) << 1) - 1u, (__float_as_uint(y) << 1) - 1u));
-    }
-}
 
 // Column layouts (CL) of a wave's two 32-column blocks: 0 the even and the odd
 // columns of its 64 (a lane then holds column pairs), 1 its two halves of 32,
@@ -205,14 +165,6 @@ struct TileShape {
     static constexpr int DEPTH = MB == 1 ? 2 : 1;
     static_assert(UA >= 1 && UB >= 1, "a K-step must split evenly over the threads");
 };
-
-// An address that is the same in every lane, in scalar registers.
-__device__ __forceinline__ const float *uniform(const float *ptr) {
-    const uint64_t a = reinterpret_cast<uint64_t>(ptr);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-    return reinterpret_cast<const float *>((uint64_t)hi << 32 | lo);
-}
 
 // One operand's share of a thread: UNITS units of E consecutive k of one row
 // or column. KM: stored k-major (A of tn, B of nn and tn).

@@ -1,0 +1,60 @@
+// f32 values as exact sums of three bf16 values, for products on the bf16
+// matrix cores (gemm_split.hip says why and how exact; attention_split.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <utility>
+
+namespace mmh {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// Calls f(integral_constant<int, i>) for i = 0..n-1, so that i is a
+// compile-time constant in each call (register-slot indices stay static).
+template <class F, int... Is>
+__device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, Is...>) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+
+// Below this (2 * bits - 1 of 2^-102) a non-zero value's pieces may be
+// subnormal in bf16.
+constexpr uint32_t kTiny = 0x18ffffffu;
+
+// (bf16(x), bf16(y)), rounded to nearest even. As assembly because from the
+// cast the compiler converts x a second time on its own for the remainder.
+__device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
+    uint32_t r;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+
+// E values of consecutive k as three pieces of E bf16 each; tiny follows the
+// smallest 2 * |bits| - 1 (zeros wrap to the largest).
+template <int E>
+__device__ __forceinline__ void split_values(const float (&v)[E], uint32_t (&o)[3][E / 2],
+                                             uint32_t &tiny) {
+#pragma unroll
+    for (int i = 0; i < E / 2; ++i) {
+        const float x = v[2 * i], y = v[2 * i + 1];
+        const uint32_t h = pack_bf16(x, y);
+        const float rx = x - __uint_as_float(h << 16), ry = y - __uint_as_float(h & 0xffff0000u);
+        const uint32_t m = pack_bf16(rx, ry);
+        const float sx = rx - __uint_as_float(m << 16), sy = ry - __uint_as_float(m & 0xffff0000u);
+        o[0][i] = h;
+        o[1][i] = m;
+        o[2][i] = pack_bf16(sx, sy);
+        tiny = min(tiny, min((__float_as_uint(x) << 1) - 1u, (__float_as_uint(y) << 1) - 1u));
+    }
+}
+
+// An address that is the same in every lane, in scalar registers.
+__device__ __forceinline__ const float *uniform(const float *ptr) {
+    const uint64_t a = reinterpret_cast<uint64_t>(ptr);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return reinterpret_cast<const float *>((uint64_t)hi << 32 | lo);
+}
+
+}  // namespace mmh

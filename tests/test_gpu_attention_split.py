@@ -1,0 +1,83 @@
+"""GPU checks of the split-bf16 attention forward (attention_split.hip: heads
+of 64 and 128) against 64-bit softmax attention.
+
+Bound: a score is a sum of hd products whose six parts are each rounded into
+the sum (6 * hd / 16 roundings below 2^-23 of the absolute sum, here at most
+~6 sqrt(hd) times the scale: 2e-5), so a probability is off by at most ~2e-5 of
+itself; the output is a weighted mean of V with weights of that accuracy:
+|err| <= 4e-5 max|v|, measured two orders below.
+"""
+import numpy as np
+import pytest
+
+import midman_hip as mh
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, k, v):
+    B, H, T, hd = q.shape
+    out = np.empty(q.shape)
+    mask = np.tril(np.ones((T, T), bool))
+    for b in range(B):
+        for h in range(H):
+            j = h // (H // k.shape[1])
+            s = q[b, h].astype(np.float64) @ k[b, j].astype(np.float64).T / np.sqrt(hd)
+            s = np.where(mask, s, -np.inf)
+            e = np.exp(s - s.max(-1, keepdims=True))
+            with np.errstate(invalid="ignore"):
+                out[b, h] = (e / e.sum(-1, keepdims=True)) @ v[b, j].astype(np.float64)
+    return out
+
+
+def attend(ctx, q, k, v):
+    dev = [ctx.to_device(x) for x in (q, k, v)]
+    return mh.causal_attention(ctx, *dev).numpy()
+
+
+def inputs(B, H, Hkv, T, hd, seed):
+    r = np.random.default_rng(seed)
+    f = lambda h: r.standard_normal((B, h, T, hd), dtype=np.float32)  # noqa: E731
+    return f(H), f(Hkv), f(Hkv)
+
+
+# heads of 64 take this kernel from one 128-row block per CU on (256 blocks)
+@pytest.mark.parametrize("B,H,Hkv,hd", [(1, 4, 2, 128), (16, 16, 8, 64)])
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 96, 97, 127, 128, 129, 200, 257])
+def test_sequence_edges(ctx, B, H, Hkv, hd, T):
+    print(f"\n[attention split] B={B} H={H}/{Hkv} T={T} hd={hd}", flush=True)
+    q, k, v = inputs(B, H, Hkv, T, hd, T)
+    err = np.abs(attend(ctx, q, k, v) - reference(q, k, v)).max()
+    print(f"  max|diff| {err:.3g}", flush=True)
+    assert err <= 4e-5 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("B,H,Hkv,hd", [(1, 4, 2, 128), (16, 16, 8, 64)])
+def test_values_the_pieces_do_not_hold(ctx, B, H, Hkv, hd):
+    T = 150
+    print(f"\n[attention split] special values, hd={hd}", flush=True)
+    q, k, v = inputs(B, H, Hkv, T, hd, 9)
+    want = reference(q, k, v)
+    # V around 2^-120: its low pieces would be subnormal
+    small = np.float32(2.0**-120)
+    got = attend(ctx, q, k, v * small).astype(np.float64) / float(small)
+    assert np.abs(got - want).max() <= 4e-5 * np.abs(v).max()
+    # queries of 2^100 beside keys of 2^-100
+    got = attend(ctx, q * np.float32(2.0**100), k * np.float32(2.0**-100), v)
+    assert np.abs(got - want).max() <= 4e-5 * np.abs(v).max()
+    # an infinite value reaches the queries from its key on, in its column alone
+    w = v.copy()
+    w[:, :, 70, 3] = np.inf
+    got = attend(ctx, q, k, w)
+    assert np.all(got[:, :, 70:, 3] == np.inf)
+    keep = np.ones(got.shape, bool)
+    keep[:, :, 64:, 3] = False
+    assert np.abs(got - want)[keep].max() <= 4e-5 * np.abs(v).max()
+    # a NaN query row stays alone
+    w = q.copy()
+    w[:, :, 40, 0] = np.nan
+    got = attend(ctx, w, k, v)
+    assert np.all(np.isnan(got[:, :, 40]))
+    keep = np.ones(T, bool)
+    keep[40] = False
+    assert np.abs(got - want)[:, :, keep].max() <= 4e-5 * np.abs(v).max()
