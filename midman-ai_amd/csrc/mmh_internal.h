@@ -222,10 +222,13 @@ void launch_embedding_backward(Context &ctx, const float *g, int64_t d, const in
                                const int32_t *start, const int32_t *order, int64_t n_unique,
                                float *table, bool accumulate);
 void launch_fill(Context &ctx, float *x, int64_t n, float v);
-void launch_unpack_cols(Context &ctx, const float *src, int64_t ld_src, int64_t col_off,
-                        int64_t rows, int64_t cols, float *dst);
-void launch_unpack_gate_up(Context &ctx, const float *src, int64_t rows, int64_t ff,
-                           int64_t ff_pad, float *wg, float *wu);
+// A model's device layout beside the reference's parameter order; dev_block
+// and block_params: floats of a block in each.
+struct RefLayout {
+    int64_t vocab, d, kv, ff, ff_pad, layers, block_params, dev_block, n_params;
+};
+// ref (n_params floats, the reference order) from dev (the device layout).
+void launch_gather_ref(Context &ctx, const RefLayout &p, const float *dev, float *ref);
 int64_t global_norm_scratch_bytes();
 void launch_global_norm(Context &ctx, const float *g, int64_t n, double *scratch, float *norm);
 struct AdamArgs {

@@ -399,30 +399,8 @@ struct Model {
         if (!cfg.tie) copy(dev + off_final_norm() + d, rf + d, d * V);
     }
     void dev_to_ref(const float *dev, float *ref) {
-        const int64_t d = cfg.d, kv = cfg.kv(), ff = cfg.ff, V = cfg.vocab, qc = qkv_cols();
-        auto copy = [&](float *dst, const float *src, int64_t n) {
-            check_hip(hipMemcpyAsync(dst, src, (size_t)n * 4, hipMemcpyDeviceToDevice,
-                                     ctx->stream),
-                      "weights copy");
-        };
-        copy(ref, dev, V * d);
-        for (int64_t l = 0; l < cfg.layers; ++l) {
-            float *r = ref + V * d + l * cfg.block_params();
-            float *an = r, *wq = an + d, *wk = wq + d * d, *wv = wk + d * kv;
-            float *wo_ = wv + d * kv, *mn = wo_ + d * d, *wg = mn + d, *wu = wg + d * ff;
-            float *wd_ = wu + d * ff;
-            copy(an, dev + off_block(l), d);
-            launch_unpack_cols(*ctx, dev + off_wqkv(l), qc, 0, d, d, wq);
-            launch_unpack_cols(*ctx, dev + off_wqkv(l), qc, d, d, kv, wk);
-            launch_unpack_cols(*ctx, dev + off_wqkv(l), qc, d + kv, d, kv, wv);
-            copy(wo_, dev + off_wo(l), d * d);
-            copy(mn, dev + off_mlp_norm(l), d);
-            launch_unpack_gate_up(*ctx, dev + off_wgu(l), d, ff, ff_pad, wg, wu);
-            copy(wd_, dev + off_wd(l), ff * d);
-        }
-        float *rf = ref + V * d + cfg.layers * cfg.block_params();
-        copy(rf, dev + off_final_norm(), d);
-        if (!cfg.tie) copy(rf + d, dev + off_final_norm() + d, d * V);
+        launch_gather_ref(*ctx, {cfg.vocab, cfg.d, cfg.kv(), cfg.ff, ff_pad, cfg.layers,
+                                 cfg.block_params(), dev_block(), n_params}, dev, ref);
     }
 
     // A temporary device buffer of n floats, freed when it goes out of scope
@@ -448,11 +426,20 @@ struct Model {
     }
     // A device buffer (weights or gradients) to the host in the reference order.
     void download_ref(const float *dev, float *host) {
-        DevTemp t(ctx, n_params);
-        dev_to_ref(dev, t.p);
-        check_hip(hipMemcpyAsync(host, t.p, (size_t)n_params * 4, hipMemcpyDeviceToHost,
-                                 ctx->stream),
-                  "download");
+        // The staging buffer: the context's workspace for operations up to 64
+        // MiB (an allocation and its release per call took as long as a small
+        // model's copy), a temporary above.
+        const size_t bytes = (size_t)n_params * 4;
+        std::unique_ptr<DevTemp> t;
+        float *ref;
+        if (bytes <= (size_t(64) << 20)) {
+            ref = static_cast<float *>(ctx->workspace(2, bytes));
+        } else {
+            t = std::make_unique<DevTemp>(ctx, n_params);
+            ref = t->p;
+        }
+        dev_to_ref(dev, ref);
+        check_hip(hipMemcpyAsync(host, ref, bytes, hipMemcpyDeviceToHost, ctx->stream), "download");
         check_hip(hipStreamSynchronize(ctx->stream), "download sync");
     }
 

@@ -456,52 +456,45 @@ __global__ __launch_bounds__(256) void fill_kernel(float *__restrict__ x, int64_
         x[i] = v;
 }
 
-// ---- weight-gradient unpacking ------------------------------------------------------
-__global__ __launch_bounds__(256) void unpack_cols_kernel(const float *__restrict__ src,
-                                                          int64_t ld_src, int64_t col_off,
-                                                          int64_t rows, int64_t cols,
-                                                          float *__restrict__ dst, int vec) {
-    const int64_t step = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-        const float *s = src + r * ld_src + col_off;
-        float *d = dst + r * cols;
-        if (vec) {
-            for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < cols / 4; q += step)
-                reinterpret_cast<float4 *>(d)[q] = reinterpret_cast<const float4 *>(s)[q];
-        } else {
-            for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < cols; c += step)
-                d[c] = s[c];
-        }
-    }
-}
-
-// src [rows, 2*ff_pad] interleaved (2f gate, 2f+1 up) -> wg, wu [rows, ff];
-// a thread moves 4 columns f of both.
-__global__ __launch_bounds__(256) void unpack_gate_up_kernel(const float *__restrict__ src,
-                                                             int64_t rows, int64_t ff,
-                                                             int64_t ff_pad,
-                                                             float *__restrict__ wg,
-                                                             float *__restrict__ wu, int vec) {
-    const int64_t step = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-        const float *s = src + r * 2 * ff_pad;
-        float *g = wg + r * ff, *u = wu + r * ff;
-        for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < (ff + 3) / 4;
-             q += step) {
-            const int64_t f = 4 * q;
-            const float4 a = reinterpret_cast<const float4 *>(s)[2 * q];
-            const float4 b = reinterpret_cast<const float4 *>(s)[2 * q + 1];
-            if (vec) {
-                reinterpret_cast<float4 *>(g)[q] = make_float4(a.x, a.z, b.x, b.z);
-                reinterpret_cast<float4 *>(u)[q] = make_float4(a.y, a.w, b.y, b.w);
+// ---- parameters in the reference order ------------------------------------------------
+// One launch instead of a copy or an unpacking kernel per parameter (51 of them
+// for the tiny preset: its gradients' download 697 -> 320 us). Thread i
+// writes reference element i; the device layout is Model's (embed; per block
+// attn_norm, Wqkv, Wo, mlp_norm, Wgu with gate and up interleaved, Wd; final_norm
+// and lm_head). I: an index type that holds every count.
+template <class I>
+__global__ __launch_bounds__(256) void gather_ref_kernel(RefLayout p, const float *__restrict__ dev,
+                                                         float *__restrict__ ref) {
+    const I d = (I)p.d, kv = (I)p.kv, ff = (I)p.ff, qc = d + 2 * kv, embed = (I)(p.vocab * p.d);
+    const I blocks = (I)p.layers * (I)p.block_params, n = (I)p.n_params;
+    for (I i = (I)blockIdx.x * 256 + threadIdx.x; i < n; i += (I)gridDim.x * 256) {
+        I src = i;
+        if (i >= embed + blocks) {
+            src = embed + (I)p.layers * (I)p.dev_block + (i - embed - blocks);
+        } else if (i >= embed) {
+            const I l = (i - embed) / (I)p.block_params;
+            I r = (i - embed) - l * (I)p.block_params;
+            src = embed + l * (I)p.dev_block;
+            const I gu = d + d * qc + d * d + d;  // Wgu's place in a block
+            if (r < d) {
+                src += r;
+            } else if ((r -= d) < d * d) {
+                src += d + r / d * qc + r % d;
+            } else if ((r -= d * d) < d * kv) {
+                src += d + r / kv * qc + d + r % kv;
+            } else if ((r -= d * kv) < d * kv) {
+                src += d + r / kv * qc + d + kv + r % kv;
+            } else if ((r -= d * kv) < d * d + d) {  // Wo and mlp_norm
+                src += d + d * qc + r;
+            } else if ((r -= d * d + d) < d * ff) {
+                src += gu + r / ff * (2 * (I)p.ff_pad) + 2 * (r % ff);
+            } else if ((r -= d * ff) < d * ff) {
+                src += gu + r / ff * (2 * (I)p.ff_pad) + 2 * (r % ff) + 1;
             } else {
-                const float gv[4] = {a.x, a.z, b.x, b.z}, uv[4] = {a.y, a.w, b.y, b.w};
-                for (int j = 0; j < 4 && f + j < ff; ++j) {
-                    g[f + j] = gv[j];
-                    u[f + j] = uv[j];
-                }
+                src += gu + 2 * d * (I)p.ff_pad + (r - d * ff);
             }
         }
+        ref[i] = dev[src];
     }
 }
 
@@ -772,27 +765,16 @@ void launch_fill(Context &ctx, float *x, int64_t n, float v) {
     check_hip(hipGetLastError(), "fill launch");
 }
 
-void launch_unpack_cols(Context &ctx, const float *src, int64_t ld_src, int64_t col_off,
-                        int64_t rows, int64_t cols, float *dst) {
-    const int vec = cols % 4 == 0 && ld_src % 4 == 0 && col_off % 4 == 0 && al16(src) && al16(dst);
-    const int64_t units = vec ? cols / 4 : cols;
-    const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>((units + 255) / 256, 64)),
-                    (unsigned)std::max<int64_t>(1, std::min<int64_t>(rows, 65535)));
-    hipLaunchKernelGGL(unpack_cols_kernel, grid, dim3(256), 0, ctx.stream, src, ld_src, col_off,
-                       rows, cols, dst, vec);
-    check_hip(hipGetLastError(), "unpack launch");
-}
-
-void launch_unpack_gate_up(Context &ctx, const float *src, int64_t rows, int64_t ff,
-                           int64_t ff_pad, float *wg, float *wu) {
-    if (ff_pad % 4 || ff_pad < ff || !al16(src))
-        fail(MMH_ERR_ARGUMENT, "unpack: padded rows must be float4s");
-    const int vec = ff % 4 == 0 && al16(wg) && al16(wu);
-    const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(((ff + 3) / 4 + 255) / 256, 64)),
-                    (unsigned)std::max<int64_t>(1, std::min<int64_t>(rows, 65535)));
-    hipLaunchKernelGGL(unpack_gate_up_kernel, grid, dim3(256), 0, ctx.stream, src, rows, ff,
-                       ff_pad, wg, wu, vec);
-    check_hip(hipGetLastError(), "unpack launch");
+void launch_gather_ref(Context &ctx, const RefLayout &p, const float *dev, float *ref) {
+    const unsigned blocks = (unsigned)std::min<int64_t>((p.n_params + 255) / 256, 1 << 20);
+    // (the last step of a thread's index must not wrap)
+    if (p.n_params + (int64_t)blocks * 256 < (int64_t(1) << 32))
+        hipLaunchKernelGGL(gather_ref_kernel<uint32_t>, dim3(blocks), dim3(256), 0, ctx.stream, p,
+                           dev, ref);
+    else
+        hipLaunchKernelGGL(gather_ref_kernel<uint64_t>, dim3(blocks), dim3(256), 0, ctx.stream, p,
+                           dev, ref);
+    check_hip(hipGetLastError(), "reference order launch");
 }
 
 int64_t global_norm_scratch_bytes() { return (int64_t)NORM_BLOCKS * 8; }
