@@ -22,11 +22,15 @@ __device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, Is.
 // subnormal in bf16.
 constexpr uint32_t kTiny = 0x18ffffffu;
 
-// (bf16(x), bf16(y)), rounded to nearest even. As assembly because from the
-// cast the compiler converts x a second time on its own for the remainder.
+// (bf16(x), bf16(y)), rounded to nearest even. The empty assembly hides where r
+// comes from: without it the compiler converts x a second time on its own for
+// the remainder. The instruction itself stays the compiler's, which has to keep
+// two wait states between it and a matrix instruction that reads r.
 __device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
-    uint32_t r;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    typedef float floatx2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    uint32_t r = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x, y}, bf16x2));
+    asm("" : "+v"(r));
     return r;
 }
 
