@@ -22,8 +22,8 @@ LIB = os.path.join(HERE, "libmidman_hip.so")
 ARCH = "gfx950"
 
 HIP_SOURCES = ["gemm_split.hip", "gemm.hip", "runtime.hip", "rowops.hip",
-               "attention.hip", "attention_split.hip", "attention_bwd.hip", "train.hip",
-               "checkpoint.hip", "model.hip", "noalloc.hip", "fused_forward.hip"]
+               "attention.hip", "attention_split.hip", "attention_bwd.hip",
+               "attention_bwd_split.hip", "train.hip", "checkpoint.hip", "model.hip", "noalloc.hip", "fused_forward.hip"]
 # Host code with no HIP in it (also built with the sanitizers: build_sanitized.py)
 HOST_SOURCES = ["host_errors.cpp", "host_math.cpp", "host_sha256.cpp", "host_safetensors.cpp",
                 "host_data.cpp"]

@@ -30,26 +30,18 @@
 // second kernel sums a group's partials in head order. The gradient of
 // the scaled scores is dS*scale (attention.rs:83), applied to dQ and dK at
 // the end. Entries above the diagonal have P = 0 and contribute nothing.
-// Heads of 64 and 128 take the same products with 16 rows per wave
+// Heads of 64 and 128 take the same products on the bf16 matrix cores
+// (attention_bwd_split.hip) or, for short sequences, with 16 rows per wave
 // (attn_bwd_dq16_kernel, attn_bwd_dkv16_kernel below); small grids take the
 // strip kernels at the end of the file.
 #include <algorithm>
 
-#include "mmh_internal.h"
+#include "mmh_attention.h"
 
 namespace mmh {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-struct BwdP {
-    const float *q, *k, *v, *o, *dout, *lse;
-    float *dq, *dk, *dv, *dvec;
-    int64_t sqb, sqh, sqt, skb, skh, skt, svb, svh, svt, sob, soh, sot;
-    float *part;  // per-query-head partial dK, dV [2][B][H][T][hd], or null
-    int h, hkv, t, nqb, nkb;
-    float scale;
-};
 
 // A raw buffer over everything from base on (32-bit offsets, no range
 // check that matters) and its 16-byte load.
@@ -1187,6 +1179,13 @@ void backward_kernels(Context &ctx, const AttnBwdDesc &d, float scale) {
     const int64_t span = d.t * std::max(std::max(d.sqt, d.skt), std::max(d.svt, d.sot)) +
                          d.h * std::max(d.sqh, d.soh) + d.hd;
     const bool off32 = span < (int64_t(1) << 29);
+    // Of those, the bf16-piece kernels (attention_bwd_split.hip) from 200
+    // positions at heads of 64 and from 64 at heads of 128. Below that a
+    // workgroup of theirs has too few tiles to make up for its setup and for
+    // being alone on its CU: B64 16/8 heads of 64, whole backward, 16-row
+    // kernels against pieces: T64 98 / 116 us, T128 190 / 191, T192 347 / 359,
+    // T224 443 / 414, T1000 (B4 12/12) 308 / 197; B32 16/8 heads of 128: T32
+    // 65 / 69, T64 105 / 104, T128 195 / 184, T200 439 / 359.
 #define MMH_BWD_CASE(HD)                                                                   \
     case HD:                                                                               \
         if constexpr (HD <= 64) {                                                          \
@@ -1198,6 +1197,10 @@ void backward_kernels(Context &ctx, const AttnBwdDesc &d, float scale) {
         }                                                                                  \
         if constexpr (HD == 64 || HD == 128) {                                             \
           if (off32) {                                                                     \
+            if (d.t >= (HD == 64 ? 200 : 64)) {                                            \
+                launch_attention_bwd_split(ctx, p, d.b, HD);                               \
+                break;                                                                     \
+            }                                                                              \
             hipLaunchKernelGGL((attn_bwd_dq16_kernel<HD>), gq, dim3(512), 0, ctx.stream, p);  \
             hipLaunchKernelGGL((attn_bwd_dkv16_kernel<HD>), gk, dim3(512), 0, ctx.stream, p); \
             break;                                                                         \
