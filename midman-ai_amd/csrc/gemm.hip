@@ -758,6 +758,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_mfma_ksplit(KParams p) {
     if (split_last(p, tm * p.tiles_n + tn)) split_reduce_tile(p, m0, n0, 32, 32, 64 * NW);
 }
 
+// Waves of a K-split workgroup: one per K step of a split, in multiples of four
+// (one per SIMD) up to sixteen: a wave that walked two steps would wait on its
+// second step's loads after its first step's MFMAs, and the others on it.
+int ksplit_waves(int64_t steps) { return steps <= 4 ? 4 : steps <= 8 ? 8 : steps <= 12 ? 12 : 16; }
+
 template <bool TA, bool TB, int EPI, bool NORM, int MODE>
 void launch_ksplit_mode(Context &ctx, const KParams &p, dim3 grid, int nw) {
     if (nw == 4)
@@ -784,13 +789,9 @@ void launch_ksplit_nw(Context &ctx, const KParams &p, dim3 grid, int mode, int n
         launch_ksplit_mode<TA, TB, EPI, NORM, 0>(ctx, p, grid, nw);
 }
 
-// One wave per K step of a split, in multiples of four waves (one per SIMD)
-// up to sixteen: a wave that walked two steps would wait on its second
-// step's loads after its first step's MFMAs, and the others on it.
 template <bool TA, bool TB, int EPI>
 void launch_ksplit(Context &ctx, const KParams &p, dim3 grid, int mode) {
-    const int64_t steps = (p.k_per_split + 31) / 32;
-    const int nw = steps <= 4 ? 4 : steps <= 8 ? 8 : steps <= 12 ? 12 : 16;
+    const int nw = ksplit_waves((p.k_per_split + 31) / 32);
     if constexpr (!TA && !TB && (EPI == EPI_STORE || EPI == EPI_SWIGLU)) {
         if (p.norm_w) {
             launch_ksplit_nw<false, false, EPI, true>(ctx, p, grid, mode, nw);
@@ -899,6 +900,35 @@ int ksplit_kind(const Context &ctx, const GemmDesc &d) {
         !d.rope_cos && big_tiles < cus && d.m * d.n * d.k <= (int64_t(1) << 28))
         return 2;
     return 0;
+}
+
+// K splits of a kind-2 K-split product: the least estimated time, in ns. A CU
+// holds 16 waves; a round of steps on all of them takes about 4.2 us, on 8
+// waves 3.2 (loads in flight, then the MFMAs); the splits' partials meet in
+// memory for 1.2 us and 0.35 more per split. (It was two workgroups per CU with
+// as few as four steps each: tn 128x384x2048 13.8 us, 8.8 by this estimate,
+// 344x128x2048 13.6 / 8.7, 96x96x1024 8.2 / 6.3, 128x128x8192 18.8 / 13.3,
+// 2048x128x688 (not split any more) 14.5 / 8.7, 128x688x2048 14.5 / 14.4.)
+// uncoalesced: both operands k-major and not 16-byte aligned, read one value
+// per lane and row: the rows' cache lines bound it, and many small workgroups
+// spread them (nt 574x51x723 10.6 us so, 12.6 by the estimate).
+int ksplit_splits(int cus, int64_t tiles, int64_t ktiles, bool uncoalesced) {
+    int best = 1;
+    if (uncoalesced) {
+        while (tiles * best < 2 * (int64_t)cus && best < 64 && ktiles / (best * 2) >= 4) best *= 2;
+        return best;
+    }
+    int64_t least = INT64_MAX;
+    for (int s = 1; s <= 64 && (s == 1 || ktiles / s >= 8); s *= 2) {
+        const int64_t steps = (ktiles + s - 1) / s, nw = ksplit_waves(steps);
+        const int64_t wgs = cus * (16 / nw), rounds = (tiles * s + wgs - 1) / wgs * ((steps + nw - 1) / nw);
+        const int64_t cost = rounds * (2200 + 125 * nw) + (s > 1 ? 1200 + 350 * s : 0);
+        if (cost < least) {
+            least = cost;
+            best = s;
+        }
+    }
+    return best;
 }
 
 bool vec_a_of(const GemmDesc &d, const float *a, int64_t lda) {
@@ -1138,10 +1168,7 @@ void gemm(Context &ctx, const GemmDesc &d) {
     if (tiled) {
         splits = plan.splits;
     } else if (kind == 2) {
-        // Up to two workgroups per CU, each split keeping >= 4 steps of 32
-        // (a step per wave at least).
-        while (tiles * splits < 2 * (int64_t)cus && splits < 64 && ktiles / (splits * 2) >= 4)
-            splits *= 2;
+        splits = ksplit_splits(cus, tiles, ktiles, !d.ta && d.tb && !(p.vec_a && p.vec_b));
     } else if (!ksplit && d.batch == 1 && d.epi != EPI_SWIGLU && d.epi != EPI_SWIGLU_BWD) {
         // Split only while a split keeps >= 8 steps of 32 (the reduce
         // launch costs about what 8 steps do) and the grid is below a

@@ -113,3 +113,25 @@ def test_special_values(ctx, what, m, k, n, form):
     b2 = np.abs(np.where(np.isfinite(b), b, 1)).astype(np.float32) + 1
     acc = run(ctx, form, a, b2, c0)
     assert np.all(np.signbit(acc[m // 4])) and np.all(acc[m // 4] == 0.0)
+
+
+# small products, 32x32 tiles with K split over waves and workgroups: the K
+# around a split's 8 and 16 steps, more than one step per wave, more tiles than
+# CUs, rows that are not 16-byte aligned (summed by fp32 MFMAs: one rounding
+# of at most 2^-24 of the absolute sum per value, and one per split)
+@pytest.mark.parametrize("m,k,n", [(33, 255, 31), (64, 512, 96), (64, 513, 96), (96, 1024, 96), (128, 2016, 384),
+                                   (32, 8192, 32), (512, 1600, 320), (1435, 295, 187), (560, 1168, 174),
+                                   (92, 1175, 135)])
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+def test_small_product_splits(ctx, m, k, n, form):
+    print(f"\n[gemm K split] {form} {m}x{k}x{n}", flush=True)
+    r = np.random.default_rng(m + k + n)
+    a, b = r.standard_normal((m, k), dtype=np.float32), r.standard_normal((k, n), dtype=np.float32)
+    c0 = r.standard_normal((m, n), dtype=np.float32)
+    for c in (None, c0):
+        out = run(ctx, form, a, b, c)
+        want = a.astype(np.float64) @ b.astype(np.float64) + (0 if c is None else c)
+        size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64) + (0 if c is None else np.abs(c))
+        worst = float((np.abs(out - want) / ((k + 64) * 2.0**-24 * size)).max())
+        print(f"  max err / bound {worst:.3g}", flush=True)
+        assert worst <= 1.0
