@@ -83,6 +83,8 @@ struct Context {
     // with the context.
     static constexpr int kTickets = 4096;
     int32_t *tickets = nullptr;
+    // Two words of pinned host memory for results read back (one thread per context).
+    float *words = nullptr;
     // Allocations made through mmh_alloc, freed at destroy.
     std::vector<void *> owned;
 
@@ -229,6 +231,8 @@ struct RefLayout {
 };
 // ref (n_params floats, the reference order) from dev (the device layout).
 void launch_gather_ref(Context &ctx, const RefLayout &p, const float *dev, float *ref);
+// host[0] = *a, host[1] = *b (host: pinned memory), bit for bit.
+void launch_copy_words(Context &ctx, const float *a, const float *b, float *host);
 int64_t global_norm_scratch_bytes();
 void launch_global_norm(Context &ctx, const float *g, int64_t n, double *scratch, float *norm);
 struct AdamArgs {

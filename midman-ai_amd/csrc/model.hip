@@ -568,19 +568,45 @@ struct Model {
     // no fused launch ran); waits for queued work. A nonzero word is cleared
     // together with the counters, so the next launch starts clean.
     int32_t take_fused_error() {
-        if (!fused_check || !fused_arena) return 0;
-        const FusedLayout f = fused_layout(fused_shape(fused_b, fused_t));
-        int32_t e = 0;
-        check_hip(hipMemcpyAsync(&e, fused_arena + f.o_err, 4, hipMemcpyDeviceToHost, ctx->stream),
-                  "fused error word");
-        check_hip(hipStreamSynchronize(ctx->stream), "fused error sync");
+        const float *word = fused_error_word();
+        if (!word) return 0;
+        float v[2];
+        read_words(word, word, v);
+        return settle_fused_error(v[0]);
+    }
+    const float *fused_error_word() {
+        if (!fused_check || !fused_arena) return nullptr;
+        return fused_arena + fused_layout(fused_shape(fused_b, fused_t)).o_err;
+    }
+    // The error word as read; clears it.
+    int32_t settle_fused_error(float v) {
+        int32_t e;
+        std::memcpy(&e, &v, 4);
         fused_check = false;
         if (e == 0) return 0;
+        const FusedLayout f = fused_layout(fused_shape(fused_b, fused_t));
         check_hip(hipMemsetAsync(fused_arena + f.o_ctl, 0, (size_t)f.ctl_ints * 4, ctx->stream),
                   "fused reset");
         check_hip(hipMemsetAsync(fused_arena + f.o_err, 0, 4, ctx->stream), "fused reset");
         check_hip(hipStreamSynchronize(ctx->stream), "fused reset sync");
         return e;
+    }
+    // Two device words to the host, after the queued work: one launch that
+    // writes them into the context's pinned words, one wait. (A copy of each into the
+    // caller's pageable memory waited for the stream by itself.)
+    void read_words(const float *a, const float *b, float (&out)[2]) {
+        launch_copy_words(*ctx, a, b, ctx->words);
+        check_hip(hipStreamSynchronize(ctx->stream), "result sync");
+        out[0] = ctx->words[0];
+        out[1] = ctx->words[1];
+    }
+    // The loss and the fused launches' error bits (0: none).
+    int32_t read_loss_and_error(float *out) {
+        const float *err = fused_error_word();
+        float v[2];
+        read_words(loss, err ? err : loss, v);
+        *out = v[0];
+        return err ? settle_fused_error(v[1]) : 0;
     }
     // When the fused launch of the last loss-only forward (batch x seq) gave
     // up (a dependency wait past its bound: the team's workgroups were not all
@@ -589,7 +615,9 @@ struct Model {
     // which are still in HBM; the loss buffer then holds its loss. True when
     // that happened. Waits for queued work.
     bool redo_if_fused_failed(int64_t batch, int64_t seq) {
-        const int32_t e = take_fused_error();
+        return redo_fused(take_fused_error(), batch, seq);
+    }
+    bool redo_fused(int32_t e, int64_t batch, int64_t seq) {
         if (e == 0) return false;
         fused_last_error = e;
         ++fused_fallbacks;
@@ -870,16 +898,10 @@ struct Model {
     // The loss of the last staged run (read_loss): a fused run that gave up is
     // redone on the per-operation kernels first.
     void read_staged_loss(float *out) {
-        check_hip(hipMemcpyAsync(out, loss, 4, hipMemcpyDeviceToHost, ctx->stream), "loss download");
-        check_hip(hipStreamSynchronize(ctx->stream), "loss sync");
+        const int32_t e = read_loss_and_error(out);
         if (staged_n > 0 && staged_n == run_b * run_t && staged_targets &&
-            redo_if_fused_failed(run_b, run_t)) {
-            check_hip(hipMemcpyAsync(out, loss, 4, hipMemcpyDeviceToHost, ctx->stream),
-                      "loss download");
-            check_hip(hipStreamSynchronize(ctx->stream), "loss sync");
-        } else {
-            (void)take_fused_error();
-        }
+            redo_fused(e, run_b, run_t))
+            (void)read_loss_and_error(out);
     }
 
     void run(const int32_t *inputs, const int32_t *targets, int64_t batch, int64_t seq,
@@ -887,21 +909,19 @@ struct Model {
         stage(inputs, loss_out ? targets : nullptr, batch, seq);
         enqueue(batch, seq, loss_out != nullptr, logits_out != nullptr);
         Context &c = *ctx;
-        if (loss_out)
-            check_hip(hipMemcpyAsync(loss_out, loss, 4, hipMemcpyDeviceToHost, c.stream),
-                      "loss download");
         if (logits_out)
             check_hip(hipMemcpyAsync(logits_out, logits, (size_t)(batch * seq * cfg.vocab) * 4,
                                      hipMemcpyDeviceToHost, c.stream),
                       "logits download");
-        check_hip(hipStreamSynchronize(c.stream), "forward sync");
+        int32_t e = 0;
+        if (loss_out)
+            e = read_loss_and_error(loss_out);
+        else
+            check_hip(hipStreamSynchronize(c.stream), "forward sync");
         run_b = batch;
         run_t = seq;
-        if (redo_if_fused_failed(batch, seq) && loss_out) {
-            check_hip(hipMemcpyAsync(loss_out, loss, 4, hipMemcpyDeviceToHost, c.stream),
-                      "loss download");
-            check_hip(hipStreamSynchronize(c.stream), "forward sync");
-        }
+        if (!loss_out) e = take_fused_error();
+        if (redo_fused(e, batch, seq) && loss_out) (void)read_loss_and_error(loss_out);
     }
 
     // ---------------------------------------------------------------- training
@@ -1251,11 +1271,7 @@ struct Model {
     // Reads the loss and the norm; true when both are finite.
     bool read_step(float *loss_out, float *norm_out) {
         float host[2];
-        check_hip(hipMemcpyAsync(&host[0], loss, 4, hipMemcpyDeviceToHost, ctx->stream),
-                  "loss download");
-        check_hip(hipMemcpyAsync(&host[1], tr.norm, 4, hipMemcpyDeviceToHost, ctx->stream),
-                  "norm download");
-        check_hip(hipStreamSynchronize(ctx->stream), "step sync");
+        read_words(loss, tr.norm, host);
         if (loss_out) *loss_out = host[0];
         if (norm_out) *norm_out = host[1];
         return std::isfinite(host[0]) && std::isfinite(host[1]);

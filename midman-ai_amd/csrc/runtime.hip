@@ -116,6 +116,8 @@ int32_t mmh_context_create(int32_t device, mmh_handle *out_ctx) {
         check_hip(hipMemsetAsync(c->tickets, 0, Context::kTickets * sizeof(int32_t), c->stream),
                   "ticket clear");
         check_hip(hipStreamSynchronize(c->stream), "ticket clear sync");
+        check_hip(hipHostMalloc(reinterpret_cast<void **>(&c->words), 8, hipHostMallocDefault),
+                  "result words");
         std::lock_guard<std::mutex> lock(g_mutex);
         g_contexts.push_back(std::move(c));
         *out_ctx = (mmh_handle)g_contexts.size();
@@ -139,6 +141,7 @@ int32_t mmh_context_destroy(mmh_handle ctx) {
         for (int s = 0; s < Context::kSlots; ++s)
             if (c->ws[s]) (void)hipFree(c->ws[s]);
         if (c->tickets) (void)hipFree(c->tickets);
+        if (c->words) (void)hipHostFree(c->words);
         (void)hipEventDestroy(c->t0);
         (void)hipEventDestroy(c->t1);
         (void)hipStreamDestroy(c->stream);

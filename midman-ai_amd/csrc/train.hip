@@ -428,6 +428,11 @@ __global__ __launch_bounds__(64 * SUM_WAVES) void sum_rows_kernel(const float *_
     }
 }
 
+// Two words into pinned host memory.
+__global__ void copy_words_kernel(const uint32_t *a, const uint32_t *b, uint32_t *host) {
+    if (threadIdx.x < 2) host[threadIdx.x] = threadIdx.x ? *b : *a;
+}
+
 // ---- embedding backward ----------------------------------------------------------
 // Workgroup u owns table row ids[u]: the gradient rows at positions
 // order[start[u] .. start[u+1]) are added in that (ascending) order from zero,
@@ -763,6 +768,13 @@ void launch_embedding_backward(Context &ctx, const float *g, int64_t d, const in
 void launch_fill(Context &ctx, float *x, int64_t n, float v) {
     hipLaunchKernelGGL(fill_kernel, dim3(grid_for(n)), dim3(256), 0, ctx.stream, x, n, v);
     check_hip(hipGetLastError(), "fill launch");
+}
+
+void launch_copy_words(Context &ctx, const float *a, const float *b, float *host) {
+    hipLaunchKernelGGL(copy_words_kernel, dim3(1), dim3(64), 0, ctx.stream,
+                       reinterpret_cast<const uint32_t *>(a), reinterpret_cast<const uint32_t *>(b),
+                       reinterpret_cast<uint32_t *>(host));
+    check_hip(hipGetLastError(), "result words launch");
 }
 
 void launch_gather_ref(Context &ctx, const RefLayout &p, const float *dev, float *ref) {
