@@ -24,10 +24,12 @@
  * (id < V, as ops_shape.rs:250-252 and ops_reduce.rs:250-252 do) before any
  * launch, so an out-of-range id is MMH_ERR_INDEX and nothing runs.
  *
- * Numerics: all arithmetic is IEEE f32 as in the reference; GEMM sums are
- * formed by fp32 MFMA in a different order from the reference's sequential
- * p-ascending loop, so results agree within a tolerance, not bit for bit
- * (see each function). Embedding, RoPE, token and index handling are bit-exact.
+ * Numerics: inputs, results and sums are f32 as in the reference. Products are
+ * summed on the matrix cores in a different order from the reference's
+ * sequential p-ascending loop, either in fp32 or (the larger GEMMs, attention
+ * with heads of 64 and 128) from exact splits of the f32 operands into three
+ * bf16 values, whose error is no larger; so results agree within a tolerance,
+ * not bit for bit (see each function). Embedding, RoPE, token and index handling are bit-exact.
  */
 #ifndef MIDMAN_HIP_H
 #define MIDMAN_HIP_H

@@ -112,7 +112,7 @@ Config parse_config(const double *v) {
 // SwiGLU into the gate/up GEMM, and the two norms and the q, k rotation
 // handed to the QKV and gate/up GEMMs, which fold them in where they can
 // (the norms at small widths; the rotation for heads of up to 32 columns on
-// the small tiles and of 64 or 128 on the 128x128 tiles) and run them as
+// the small tiles and of 64 or 128 on the large tiles) and run them as
 // kernels of their own otherwise. timed(class, launch) wraps each launch.
 struct BlockRun {
     const float *attn_norm = nullptr, *wqkv = nullptr, *wo = nullptr;

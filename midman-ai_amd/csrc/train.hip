@@ -11,8 +11,8 @@
 //     per workgroup into a partial row, then over workgroups in a fixed order.
 //   embedding backward (ops_shape.rs:261-269): rows of the same id are added
 //     in position order from a host-built index (no atomics).
-//   unpacking of the fused QKV and interleaved gate/up weight gradients into
-//     the reference's parameter layout.
+//   parameters or gradients in the reference's order, gathered from the device
+//     layout (fused QKV, interleaved gate/up) by one kernel.
 //   global norm (clip.rs:30-33): f64 sum of squares, fixed reduction tree.
 //   clip + AdamW (clip.rs:42-60, adamw.rs:180-214): one pass over every
 //     parameter; nothing is written when the loss or the norm is not finite.
