@@ -974,6 +974,7 @@ struct TilePlan {
 // Split partials of the large tiles stay below this: the no-alloc entry point's
 // array holds them too, so both entry points take the same plan.
 constexpr int64_t kSplitBytes = kNoallocScratchBytes;
+constexpr int kMaxTileSplits = 16;
 
 // The tile and the K splits that an estimate of the launch makes shortest: with
 // G workgroups and q = ceil(G / CUs) on the busiest CU, 16 of K take
@@ -987,30 +988,39 @@ constexpr int64_t kSplitBytes = kNoallocScratchBytes;
 // CU (1000 x 768 x 3072: 36.9 us against 40.9 and 41.8 for its neighbours),
 // 128x64 and 64x64 below (2048 x 512 x 1024 20.9 us against 32 for 128x128);
 // 1024 x 2048 x 4096 takes two splits of 256x128 (102 us against 117 whole).
+// Split counts other than 2, 4 and 8 fill the CUs that a halving leaves idle
+// (2816 x 2688 x 324: 3 splits 45 us, 2 splits 71; 976 x 3694 x 1046 65 / 91;
+// 150 x 7999 x 4224 102 / 139; 508 x 7168 x 128: 16 splits 18.3, 8 splits
+// 22.3). They are taken when the estimate is 4% lower: where it gains less,
+// half of the products measured got slower by up to 10% (919 x 7189 x 490 57 ->
+// 61, 128 x 1664 x 3648 21 -> 23). Past 8 the sums of a split's partials wait
+// on memory once more per four of them, 0.2 us each.
 TilePlan choose_tile(const Context &ctx, const KParams &p, int64_t batch, int epi) {
     const bool may_split = batch == 1 && (epi == EPI_STORE || epi == EPI_ACCUM) && !p.rope_cos;
     const double cus = cus_of(ctx), ksteps = (double)((p.k + BK - 1) / BK);
-    TilePlan best;
-    double best_us = 0.0;
+    TilePlan best[2];  // of the halvings of K, of the other split counts
+    double best_us[2] = {0.0, 0.0};
     for (int tile = 0; tile < TILE_COUNT; ++tile) {
         if (!gemm_tile_takes(p, epi, tile)) continue;
         const GemmTileInfo &t = kGemmTiles[tile];
         const double tiles = (double)((p.m + t.rows - 1) / t.rows) *
                              (double)((p.n + t.cols - 1) / t.cols) * (double)batch;
-        for (int s = 1; s <= 8; s *= 2) {
+        for (int s = 1; s <= kMaxTileSplits; ++s) {
             // a split keeps 128 of K, as many as its prologue costs
             if (s > 1 && (!may_split || p.k < 128 * s || s * p.m * p.n * 4 > kSplitBytes)) break;
             const double g = tiles * s;
             double us = std::max(std::ceil(g / cus) * t.alone, g / cus * t.full) * (ksteps / s + 6.0);
             if (s > 1) us += 4.0 + (double)(s + 1) * (double)(p.m * p.n) * 4.0 / 4.5e6;
-            if (best_us == 0.0 || us < best_us) {
-                best_us = us;
-                best.tile = tile;
-                best.splits = s;
+            if (s > 8) us += 0.2 * (s - 8);
+            const int fine = s > 8 || (s & (s - 1)) ? 1 : 0;
+            if (best_us[fine] == 0.0 || us < best_us[fine]) {
+                best_us[fine] = us;
+                best[fine].tile = tile;
+                best[fine].splits = s;
             }
         }
     }
-    return best;
+    return best_us[1] > 0.0 && best_us[1] < 0.96 * best_us[0] ? best[1] : best[0];
 }
 
 // mmh_gemm_noalloc's contract: which products it takes is stated in terms of a

@@ -4,7 +4,8 @@ bf16 MFMA products of exact three-way splits, against 64-bit sums.
 Bound per element: with S = sum_p |a_p b_p|, the three products left out are
 below 3 * 2^-24 S; the matrix core rounds the running sum once per product
 group of 16 k, six groups per 16 k, each below 2^-23 S (it may truncate); a K
-split adds at most 8 partials. So |err| <= (6 * ceil(k / 16) + 16) * 2^-23 * S.
+split adds at most 16 partials, a rounding of 2^-24 each. So |err| <=
+(6 * ceil(k / 16) + 16) * 2^-23 * S.
 """
 import numpy as np
 import pytest
@@ -24,6 +25,8 @@ SHAPES = [
     ("128x64, an odd step", 2000, 528, 1001),
     ("64x64, 4 wave groups, 3 odd steps and a tail", 1030, 569, 515),
     ("64x64 in splits", 300, 5003, 301),
+    ("128x128 in 3 splits", 767, 1598, 1373),
+    ("64x64 in 16 splits", 130, 9001, 257),
     ("64x64, fewer whole steps than wave groups", 2300, 50, 2301),
 ]
 
@@ -120,7 +123,7 @@ def test_special_values(ctx, what, m, k, n, form):
 # CUs, rows that are not 16-byte aligned (summed by fp32 MFMAs: one rounding
 # of at most 2^-24 of the absolute sum per value, and one per split)
 @pytest.mark.parametrize("m,k,n", [(33, 255, 31), (64, 512, 96), (64, 513, 96), (96, 1024, 96), (128, 2016, 384),
-                                   (32, 8192, 32), (512, 1600, 320), (1435, 295, 187), (560, 1168, 174),
+                                   (32, 8192, 32), (2368, 3480, 32), (512, 1600, 320), (1435, 295, 187), (560, 1168, 174),
                                    (92, 1175, 135)])
 @pytest.mark.parametrize("form", ["nn", "nt", "tn"])
 def test_small_product_splits(ctx, m, k, n, form):
