@@ -647,22 +647,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_mfma_ksplit(KParams p) {
         }
     }
 
-    // Each step sums from acc_init and is then added to the wave's sum in its
-    // own LDS slots: 16 roundings at a step's size and one at the sum's, so
-    // few splits of a long K are no less precise than many (error against 64
-    // bits at 128 x 2048 x 688 1.30e-7 in 8 splits, 1.66e-7 in one, 1.34e-7 so).
-    // In registers the sum costs the 16-wave workgroup its last ones (2368 x
-    // 3480 x 32 24 -> 52 us).
-    if (wave >= nsteps) {
+    // Each step sums from acc_init; a wave with more steps than one adds them
+    // up in its own LDS slots: 16 roundings at a step's size and one at the
+    // sum's, so few splits of a long K are no less precise than many (error
+    // against 64 bits at 128 x 2048 x 688 1.30e-7 in 8 splits, 1.66e-7 in one
+    // running sum, 1.34e-7 so; 15.6 us both). The sum leaves a step's
+    // registers before the next one's loads: kept across them, it cost the
+    // kernel occupancy or spills (768 x 2356 x 89 16.7 -> 35 us, 18 so).
+    floatx16 acc;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) part[wave][r][lane] = p.acc_init;
-    }
+    for (int r = 0; r < 16; ++r) acc[r] = p.acc_init;
     float ss = 0.0f;
     for (int st = wave; st < nsteps; st += NW) {
         const int64_t kb = kbeg + (int64_t)st * 32 + 16 * lk;  // this lane's first k of the step
-        floatx16 acc;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = p.acc_init;
         const bool whole = MODE == 2 || (MODE == 1 && kb + 16 <= kend);
         float a[16], b[16];
         if (!TA && whole) {
@@ -716,13 +713,21 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_mfma_ksplit(KParams p) {
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], acc, 0, 0, 0);
-        if (st != wave) {
+        if (st + NW < nsteps) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[r] = __fadd_rn(part[wave][r][lane], acc[r]);
+            for (int r = 0; r < 16; ++r) {
+                if (st != wave) acc[r] = __fadd_rn(part[wave][r][lane], acc[r]);
+                part[wave][r][lane] = acc[r];
+                acc[r] = p.acc_init;
+            }
         }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) part[wave][r][lane] = acc[r];
     }
+    if (wave + NW < nsteps) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = __fadd_rn(part[wave][r][lane], acc[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave][r][lane] = acc[r];
 
     if (NORM) {
         // this wave's share of row lr: k 0-15 of its steps in lane lr, 16-31 in lane lr+32
