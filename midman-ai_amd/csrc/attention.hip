@@ -279,6 +279,296 @@ __global__ __launch_bounds__(512) void attn_fwd_kernel(AttnP p) {
     }
 }
 
+// 16-row strips, 16 waves (heads of 64 and 128, grids of at least one
+// 128-row block per CU, short sequences whose last block is mostly empty:
+// attention_kernels). The same pairing of a long block (nqb-1-z, waves
+// 0-7) with a short one (z, waves 8-15) and the same 32-key K/V tiles shared
+// through a double-buffered LDS stage, but each wave owns 16 query rows and
+// runs 16x16x4 MFMAs, so a wave needs half the registers (at most 128: four
+// waves per SIMD instead of two). Wave w of a block takes strip w (w < 4) or
+// 11 - w, so the two waves of a block that share a SIMD (w and w + 4) hold
+// strips i and 7 - i: every SIMD carries the same causal work, and the
+// barrier that ends each tile waits for no SIMD with more tiles than another.
+// A wave stores its rows straight from its accumulators as soon as its last
+// tile is done, while the other waves still compute.
+//
+// Layouts (lane l, g = l/16, i = l%16; register r of an accumulator block is
+// row 4g + r of the 16x16 result, column i):
+//   S^T block kb (keys 16kb..16kb+15 of the tile, query q0 + i): k-step s
+//     pairs the head dims 32g + s (A: K[16kb + i][32g + s] from LDS, B: the
+//     lane's own Q[q0 + i][32g + s]); lane l's register r is key 16kb+4g+r.
+//   O^T block 4h+e (dims 64h + 4i' + e, i' = 0..15): k-step (kb, r) pairs the
+//     keys 16kb + 4g + r (A: V[16kb+4g+r][64h + 4i + e], B: the lane's own P
+//     register (kb, r)); lane l's register r' is O[q0 + i][64h + 16g + 4r' + e].
+// Row max and sum of a query meet across its four lanes (i, i+16, i+32, i+48)
+// through two lane swaps.
+template <int HD>
+__global__ __launch_bounds__(1024) void attn_fwd16_kernel(AttnP p) {
+    static_assert(HD == 64 || HD == 128, "16-row strips take heads of 64 or 128");
+    constexpr int NT = 1024;
+    constexpr int QB = 128;
+    constexpr int NS = HD / 4;      // S^T k-steps per key block (dims per lane group)
+    constexpr int NH = HD / 64;     // O^T dim halves: blocks 4h .. 4h+3
+    constexpr int KS = HD + 4;      // K row stride (16-byte rows, lanes 4 banks apart)
+    constexpr int F4 = 32 * HD / 4; // float4s per K or V tile
+    constexpr int PER = F4 / NT;    // 1 (HD 128) or 0.5 (HD 64: half the threads load)
+    constexpr int RA = 3;           // LDS operand reads in flight ahead of their MFMAs
+    // Two stages of 64 keys (two 32-key tiles each): one barrier per 64 keys.
+    // Tile kt lives in stage (kt/2)&1, rows 32*(kt&1) ...
+    __shared__ __attribute__((aligned(16))) float smem[2 * 64 * KS + 2 * 64 * HD];
+    auto Ks = [&](int kt) { return smem + ((kt >> 1) & 1) * 64 * KS + (kt & 1) * 32 * KS; };
+    auto Vs = [&](int kt) { return smem + 128 * KS + ((kt >> 1) & 1) * 64 * HD + (kt & 1) * 32 * HD; };
+
+    // the wave index through readfirstlane: uniform, so what derives from it
+    // (strip, rows, tile counts, their tests) is scalar work in scalar registers
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int g = lane >> 4, li = lane & 15;
+    const int half = wave >> 3, w8 = wave & 7;
+    const int strip = w8 < 4 ? w8 : 11 - w8;
+    const int head = blockIdx.x, b = blockIdx.y;
+    const int long_blk = p.nqb - 1 - (int)blockIdx.z;
+    const int qblk = half ? (int)blockIdx.z : long_blk;
+    const bool active = half == 0 || qblk < long_blk;  // nqb odd: the middle block once
+    const int kvh = head / (p.h / p.hkv);
+    const int T = p.t;
+    const int ntiles = min(long_blk * QB + QB - 1, T - 1) / 32 + 1;
+    const int q0 = qblk * QB + strip * 16;
+    const int my_tiles = active && q0 < T ? min(q0 + 15, T - 1) / 32 + 1 : 0;
+    const int qi = q0 + li;
+
+    const float *Q = p.q + b * p.sqb + head * p.sqh;
+    const float *K = p.k + b * p.skb + kvh * p.skh;
+    const float *V = p.v + b * p.svb + kvh * p.svh;
+
+    const float sc = p.scale * 1.4426950408889634f;  // scores in log2 units
+    float qr[NS];
+    {
+        const float4 *src = reinterpret_cast<const float4 *>(Q + (int64_t)min(qi, T - 1) * p.sqt + g * NS);
+#pragma unroll
+        for (int s = 0; s < NS / 4; ++s) {
+            const float4 v = src[s];
+            qr[4 * s + 0] = v.x * sc;
+            qr[4 * s + 1] = v.y * sc;
+            qr[4 * s + 2] = v.z * sc;
+            qr[4 * s + 3] = v.w * sc;
+        }
+    }
+
+    // thread tid loads float4 tid of the K tile and of the V tile (keys past
+    // T read row T-1: finite values whose scores are masked)
+    // (HD 64: threads past the tile read a copy of another thread's float4
+    // and do not store it, so the loads need no branch and can sit inside
+    // the MFMA stream)
+    const bool loader = PER >= 1 || tid < F4;
+    const int ltid = PER >= 1 ? tid : tid % F4;
+    const int lj = (4 * ltid) / HD, lc = (4 * ltid) % HD;
+    float4 kreg, vreg;
+    // Buffer loads over the sequence's T rows: 32-bit offsets (the 64-bit
+    // address arithmetic was a dozen VALU instructions per tile, and the VALU
+    // takes its cycles from the matrix core), keys past T read zeros (finite;
+    // their scores are masked and their P is 0). The host keeps T * stride
+    // below 2^29 floats for this kernel.
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(K), (short)0, (int)(4 * (int64_t)T * p.skt), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(V), (short)0, (int)(4 * (int64_t)T * p.svt), 0x00020000);
+    const uint32_t klane = 4u * ((uint32_t)lj * (uint32_t)p.skt + (uint32_t)lc);
+    const uint32_t vlane = 4u * ((uint32_t)lj * (uint32_t)p.svt + (uint32_t)lc);
+    const uint32_t ktile = 128u * (uint32_t)p.skt, vtile = 128u * (uint32_t)p.svt;
+    auto load_tile = [&](int kt) __attribute__((always_inline)) {
+        kreg = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rk, klane + (uint32_t)kt * ktile, 0, 0));
+        vreg = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv, vlane + (uint32_t)kt * vtile, 0, 0));
+    };
+    auto store_tile = [&](int kt) __attribute__((always_inline)) {
+        if (loader) {
+            *reinterpret_cast<float4 *>(Ks(kt) + lj * KS + lc) = kreg;
+            *reinterpret_cast<float4 *>(Vs(kt) + lj * HD + lc) = vreg;
+        }
+    };
+
+    floatx4 o[4 * NH];
+#pragma unroll
+    for (int db = 0; db < 4 * NH; ++db) o[db] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    // sum / max over a query's four lanes (i, i+16, i+32, i+48). Maxima as
+    // bare v_max_f32 / v_max3_f32: fmaxf (and med3 with +inf, which the
+    // compiler folds into it) takes a quieting max of each operand it cannot
+    // prove canonical first (lane-swapped values, selects), and scores here
+    // are finite or -inf, never NaN
+    auto vmax = [](float x, float y) __attribute__((always_inline)) {
+        float r;
+        asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+        return r;
+    };
+    auto vmax3 = [](float x, float y, float z) __attribute__((always_inline)) {
+        float r;
+        asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(y), "v"(z));
+        return r;
+    };
+    auto quad_max = [&](float v) __attribute__((always_inline)) {
+        auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = vmax(__uint_as_float(a[0]), __uint_as_float(a[1]));
+        auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return vmax(__uint_as_float(c[0]), __uint_as_float(c[1]));
+    };
+    auto quad_sum = [](float v) __attribute__((always_inline)) {
+        auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+        auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return __uint_as_float(c[0]) + __uint_as_float(c[1]);
+    };
+
+    float pv[8];  // P of the current tile
+    // scores and softmax of tile kt; the next tile's global loads (tile nxt)
+    // are issued between its first MFMAs, not all at once after the barrier
+    // V operands: 8 * NH float4 per tile, step i = NH*j + h:
+    // V[16(j/4) + 4g + j%4][64h + 4li ..], each feeding 4 MFMAs, read RA ahead;
+    // the first RA are issued before the softmax, so P.V starts without waiting
+    constexpr int NV = 8 * NH;
+    float4 vring[RA + 1];
+    auto vread = [&](int kt, int i) __attribute__((always_inline)) {
+        const int j = i / NH, h = i % NH;
+        return reinterpret_cast<const float4 *>(Vs(kt) + (16 * (j >> 2) + 4 * g + (j & 3)) * HD + 4 * li)[16 * h];
+    };
+    auto qk_softmax = [&](int kt, int nxt) __attribute__((always_inline)) {
+        const float *Kb = Ks(kt);
+        // 16 float4 K operands per tile, step i = 2t + kb: K[16kb + li][g*NS + 4t ..],
+        // each feeding 4 MFMAs. Steps go in pairs (2t, 2t+1), whose MFMAs
+        // alternate between the two accumulators (no MFMA waits on the one
+        // before it); a ring of four registers holds the pair in use and the
+        // next one, the pair after that read as soon as a pair is used.
+        floatx4 sacc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+        constexpr int NK = 2 * (NS / 4);
+        float4 ring[4];
+        auto kread = [&](int i) __attribute__((always_inline)) {
+            return reinterpret_cast<const float4 *>(Kb + (16 * (i & 1) + li) * KS + g * NS)[i >> 1];
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ring[i] = kread(i);
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+        for (int t = 0; t < NK / 2; ++t) {
+            const float4 ka = ring[(2 * t) % 4], kc = ring[(2 * t + 1) % 4];
+            sacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.x, qr[4 * t + 0], sacc[0], 0, 0, 0);
+            sacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kc.x, qr[4 * t + 0], sacc[1], 0, 0, 0);
+            sacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.y, qr[4 * t + 1], sacc[0], 0, 0, 0);
+            sacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kc.y, qr[4 * t + 1], sacc[1], 0, 0, 0);
+            sacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.z, qr[4 * t + 2], sacc[0], 0, 0, 0);
+            sacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kc.z, qr[4 * t + 2], sacc[1], 0, 0, 0);
+            sacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.w, qr[4 * t + 3], sacc[0], 0, 0, 0);
+            sacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kc.w, qr[4 * t + 3], sacc[1], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+            if (2 * t + 4 < NK) {
+                ring[(2 * t) % 4] = kread(2 * t + 4);
+                ring[(2 * t + 1) % 4] = kread(2 * t + 5);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            }
+            if (t == 0) {
+                load_tile(nxt);
+                __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < RA; ++i) vring[i] = vread(kt, i);
+        __builtin_amdgcn_sched_group_barrier(0x100, RA, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        const int k0 = kt * 32;
+        // the scores stay in the accumulator registers; diagonal and partial
+        // tiles overwrite their masked keys with -inf in place (a full tile
+        // moves nothing)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pv[j] = sacc[j >> 2][j & 3];
+        if (!(k0 + 31 <= q0 && k0 + 31 < T)) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int key = k0 + 16 * (j >> 2) + 4 * g + (j & 3);
+                pv[j] = key <= qi && key < T ? pv[j] : -INFINITY;
+            }
+        }
+        float mloc = vmax3(vmax3(vmax3(pv[0], pv[1], pv[2]), pv[3], pv[4]), pv[5], pv[6]);
+        mloc = vmax(mloc, pv[7]);
+        mloc = quad_max(mloc);
+        const bool need = mloc > m_run + 8.0f;  // lazy rescale, as attn_fwd_kernel
+        if (__any(need)) {
+            const float m_new = need ? mloc : m_run;
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            l_run *= alpha;
+#pragma unroll
+            for (int db = 0; db < 4 * NH; ++db)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[db][r] *= alpha;
+            m_run = m_new;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pv[j] = __builtin_amdgcn_exp2f(pv[j] - m_run);
+        float lsum = pv[0];
+#pragma unroll
+        for (int j = 1; j < 8; ++j) lsum += pv[j];
+        // the lane's own share: the four lanes of a query rescale together
+        // (one m_run), so their shares are summed once, when the strip ends
+        l_run += lsum;
+    };
+    auto pv_apply = [&](int kt) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            if (i + RA < NV) vring[(i + RA) % (RA + 1)] = vread(kt, i + RA);
+            const float4 v4 = vring[i % (RA + 1)];
+            const int j = i / NH, h = i % NH;
+            o[4 * h + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.x, pv[j], o[4 * h + 0], 0, 0, 0);
+            o[4 * h + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.y, pv[j], o[4 * h + 1], 0, 0, 0);
+            o[4 * h + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.z, pv[j], o[4 * h + 2], 0, 0, 0);
+            o[4 * h + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.w, pv[j], o[4 * h + 3], 0, 0, 0);
+            if (i + RA < NV) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt == my_tiles - 1) l_run = quad_sum(l_run);
+        if (kt == my_tiles - 1 && qi < T) {
+            // this strip is done: its rows leave now, straight from the accumulators
+            const float inv = 1.0f / l_run;
+            float *orow = p.out + b * p.sob + head * p.soh + (int64_t)qi * p.sot;
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    *reinterpret_cast<float4 *>(orow + 64 * h + 16 * g + 4 * r) =
+                        make_float4(o[4 * h + 0][r] * inv, o[4 * h + 1][r] * inv,
+                                    o[4 * h + 2][r] * inv, o[4 * h + 3][r] * inv);
+            if (p.lse && g == 0) p.lse[((int64_t)b * p.h + head) * T + qi] = m_run + log2f(l_run);
+        }
+    };
+
+    load_tile(0);
+    store_tile(0);
+    if (ntiles > 1) {
+        load_tile(1);
+        store_tile(1);
+    }
+    __syncthreads();
+    auto step = [&](int kt) __attribute__((always_inline)) {
+        // during tile kt, the tile two ahead goes to the other stage
+        const int nxt = min(kt + 2, ntiles - 1);  // the last steps reload a tile they never store
+        if (kt < my_tiles) {
+            qk_softmax(kt, nxt);
+            pv_apply(kt);
+        } else {
+            load_tile(nxt);
+        }
+        if (kt + 2 < ntiles) store_tile(kt + 2);
+    };
+    // one stage (two tiles) per iteration: each tile's position in the stage
+    // is then a constant, and its LDS offsets immediates
+    for (int m = 0; 2 * m < ntiles; ++m) {
+        step(2 * m);
+        if (2 * m + 1 < ntiles) {
+            step(2 * m + 1);
+            if (2 * m + 2 < ntiles) __syncthreads();
+        }
+    }
+}
+
 // Key-split variant for grids that would not cover the chip (few batch x head
 // pairs, short T: the tiny preset has 32 pairs of 256 rows). A workgroup owns
 // 32 query rows; its NWV waves (4, or 8 when a block reaches more than 4 key
@@ -503,8 +793,22 @@ void launch_hd(Context &ctx, const AttnP &p, dim3 grid, bool split, bool pieces)
     }
     grid.z = (grid.z + 1) / 2;  // query blocks in pairs
     if constexpr (HD == 64 || HD == 128) {
+        // The split-bf16 kernel, but for sequences of up to three blocks whose
+        // last one is short: it spends a whole block's time on that one (a
+        // workgroup to a CU), the 16-row kernel only the rows'. B8-15 16/8,
+        // 16-row against split: heads of 64 T48 12.4 / 15.9 us, T96 17.4 / 17.2,
+        // T144 17.0 / 22.3, T192 19.2 / 14.1, T270 22.7 / 27.0, T350 34.6 / 28.3;
+        // heads of 128 T48 20.3 / 24.2, T96 19.4 / 18.8, T144 28.4 / 34.3, T224
+        // 45.4 / 26.4, T270 40.3 / 43.3; with 800 blocks, heads of 64 T110 40.1
+        // / 42.2. From four blocks on the last one no longer matters (T1340 72.2
+        // / 72.3).
+        const int last = p.t - 128 * (p.nqb - 1);
+        const bool rows16 = p.nqb == 1 ? last <= (HD == 64 ? 112 : 64) : p.nqb <= 3 && last <= 56;
         if (pieces) {
-            launch_attention_split(ctx, p, grid.y, HD);
+            if (rows16)
+                hipLaunchKernelGGL((attn_fwd16_kernel<HD>), grid, dim3(1024), 0, ctx.stream, p);
+            else
+                launch_attention_split(ctx, p, grid.y, HD);
             return;
         }
     }

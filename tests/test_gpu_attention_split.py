@@ -41,9 +41,10 @@ def inputs(B, H, Hkv, T, hd, seed):
     return f(H), f(Hkv), f(Hkv)
 
 
-# heads of 64 take this kernel from one 128-row block per CU on (256 blocks)
+# heads of 64 take this kernel from one 128-row block per CU on (256 blocks); short
+# last blocks (up to 112 or 64 rows of one block, 56 of two or three) the 16-row one
 @pytest.mark.parametrize("B,H,Hkv,hd", [(1, 4, 2, 128), (16, 16, 8, 64)])
-@pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 96, 97, 127, 128, 129, 200, 257])
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 96, 97, 112, 113, 127, 128, 129, 184, 185, 200, 257])
 def test_sequence_edges(ctx, B, H, Hkv, hd, T):
     print(f"\n[attention split] B={B} H={H}/{Hkv} T={T} hd={hd}", flush=True)
     q, k, v = inputs(B, H, Hkv, T, hd, T)
