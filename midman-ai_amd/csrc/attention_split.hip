@@ -83,8 +83,12 @@ __device__ __noinline__ void exact_strip(const float *Q, const float *K, const f
         for (int c = 0; c < HH; ++c) s += q[c] * krow[c];
         s = swap_sum(s);
         if (key <= qi) {
+            // scores of -inf before the row's first other one have weight 0 (a
+            // row of nothing else is NaN, as inf - inf makes it)
+            const bool none = m == -INFINITY && s == -INFINITY && key < qi;
             const float m_new = fmaxf(m, s);
-            const float alpha = __builtin_amdgcn_exp2f(m - m_new), e = __builtin_amdgcn_exp2f(s - m_new);
+            const float alpha = none ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+            const float e = none ? 0.0f : __builtin_amdgcn_exp2f(s - m_new);
             l = l * alpha + e;
 #pragma unroll
             for (int c = 0; c < HH; ++c) acc[c] = acc[c] * alpha + e * vrow[c];

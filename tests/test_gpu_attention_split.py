@@ -82,3 +82,29 @@ def test_values_the_pieces_do_not_hold(ctx, B, H, Hkv, hd):
     keep = np.ones(T, bool)
     keep[40] = False
     assert np.abs(got - want)[:, :, keep].max() <= 4e-5 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("n", [1, 5, 40])
+@pytest.mark.parametrize("B,H,Hkv,hd", [(1, 4, 2, 128), (16, 16, 8, 64)])
+def test_leading_scores_of_minus_infinity(ctx, B, H, Hkv, hd, n):
+    # the first n keys score -inf for the queries from n on, from an infinite
+    # key and from a product that overflows: weight 0, as if they were masked
+    T = 200
+    print(f"\n[attention split] {n} leading scores of -inf, hd={hd}", flush=True)
+    q, k, v = inputs(B, H, Hkv, T, hd, 11)
+    q[..., 0], k[..., 0] = 0.0, 0.0
+    want = reference(q[:, :, n:], k[:, :, n:], v[:, :, n:])
+    bound = 4e-5 * np.abs(v).max()
+    for big, low in ((np.float32(1.0), -np.float32(np.inf)), (np.float32(1e20), np.float32(-1e20))):
+        w, x = q.copy(), k.copy()
+        w[:, :, n:, 0], x[:, :, :n, 0] = big, low
+        got = attend(ctx, w, x, v)
+        assert np.abs(got[:, :, n:] - want).max() <= bound
+    # (the overflowing product leaves the queries before n as they were)
+    assert np.abs(got[:, :, :n] - reference(q[:, :, :n], k[:, :, :n], v[:, :, :n])).max() <= bound
+    g = ctx.to_device(np.ones_like(q))
+    grads = mh.causal_attention_backward(ctx, *(ctx.to_device(a) for a in (w, x, v)), g)
+    assert all(np.isfinite(a.numpy()).all() for a in grads)
+    # no score but -inf: NaN
+    w[..., 0] = big
+    assert np.isnan(attend(ctx, w, x, v)[:, :, :n]).all()
