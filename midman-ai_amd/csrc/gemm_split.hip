@@ -17,12 +17,16 @@
 // 1.62e-6: a 32x32x16 step rounds the sum six times per 16 products, the
 // fp32 32x32x2 step eight times.
 //
+// The operands are lifted by 2^24 first (mmh_split.h), a multiply per value, so
+// that small values need no second look. Following the smallest magnitude
+// instead, to redo the tiles of values below 2^-102, took more (4096 x 4096 x
+// 2048 332 us, 323 so) and made such operands four to eight times slower (4096 x
+// 2048 x 8192 nt 597 -> 4800 us).
+//
 // What the split cannot hold is found and redone with the fp32 MFMA, tile by
-// tile, so special values follow the scalar rules bit for bit as before:
-//   - inf, NaN, |x| above bf16's largest finite value, and sums that overflow
+// tile, so special values follow the scalar rules bit for bit:
+//   - inf, NaN, |x| from 2^104 on (the lift, mmh_split.h) and sums from 2^80 on
 //     leave a non-finite accumulator (inf - inf in the remainders);
-//   - 0 < |x| < 2^-102, whose low pieces would leave bf16's normal range: the
-//     smallest non-zero magnitude is followed as the values are split;
 //   - an exact zero where the sum must keep the sign of -0 (acc_init is -0).
 //
 // Tiling: a wave owns MB x 2 blocks of 32x32 (MB 4: 128x64, 2: 64x64, 1:
@@ -49,7 +53,8 @@
 // reach 1730-1770 TFLOP/s = 290 in f32 terms, and 1600 with the VALU work of
 // the splits beside them. Measured at 4096 x 4096 x 2048: 256x256 311 us = 221
 // TFLOP/s, 256x128 333 us, 128x128 375 us (more LDS reads and splits per
-// product); the fp32 MFMA kernel before it 471 us = 146.
+// product); the fp32 MFMA kernel before it 471 us = 146 (before the lift; 2-3%
+// less since).
 //
 // MFMA 32x32x16 bf16 layout (wave64): lane l supplies A[i = l%32][k = 8*(l/32)
 // .. +7] and B[k = 8*(l/32) .. +7][j = l%32]; accumulator register r of lane l
@@ -234,14 +239,14 @@ struct Loader {
     }
 };
 
-// The K loop of one tile; returns the smallest 2 * |bits| - 1 this thread split.
+// The K loop of one tile; the sums it leaves are lifted twice (kUnlift2).
 // WK groups of WM x WN waves share a tile: group g takes the steps g, g + WK,
 // ... into its own LDS stages and its own accumulators.
 template <bool TA, bool TB, int CL, int WM, int WN, int MB, int WK>
-__device__ __forceinline__ uint32_t split_mainloop(const KParams &p, const float *__restrict__ A,
-                                                   const float *__restrict__ B, int64_t m0,
-                                                   int64_t n0, int64_t kbeg, int64_t kend,
-                                                   char *lds, floatx16 (&acc)[MB][2]) {
+__device__ __forceinline__ void split_mainloop(const KParams &p, const float *__restrict__ A,
+                                               const float *__restrict__ B, int64_t m0,
+                                               int64_t n0, int64_t kbeg, int64_t kend,
+                                               char *lds, floatx16 (&acc)[MB][2]) {
     using S = TileShape<WM, WN, MB>;
     constexpr int TM = S::TM, TN = S::TN, NT = S::NT;
     const int group = WK == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
@@ -281,13 +286,12 @@ __device__ __forceinline__ uint32_t split_mainloop(const KParams &p, const float
         la.load(ra[slot], k0);
         lb.load(rb[slot], k0);
     };
-    uint32_t tiny = 0xffffffffu;
     auto put = [&](int buf, int slot) __attribute__((always_inline)) {
         char *stage = lds + buf * S::STAGE;
 #pragma unroll
         for (int i = 0; i < S::UA; ++i) {
             uint32_t o[3][S::EA / 2];
-            split_values(ra[slot][i], o, tiny);
+            lift_and_split(ra[slot][i], o);
 #pragma unroll
             for (int q = 0; q < 3; ++q)
                 __builtin_memcpy(__builtin_assume_aligned(stage + q * 2 * S::PA + wa[i], S::EA * 2),
@@ -296,7 +300,7 @@ __device__ __forceinline__ uint32_t split_mainloop(const KParams &p, const float
 #pragma unroll
         for (int i = 0; i < S::UB; ++i) {
             uint32_t o[3][S::EB / 2];
-            split_values(rb[slot][i], o, tiny);
+            lift_and_split(rb[slot][i], o);
 #pragma unroll
             for (int q = 0; q < 3; ++q)
                 __builtin_memcpy(__builtin_assume_aligned(stage + q * 2 * S::PB + wb[i], S::EB * 2),
@@ -407,7 +411,7 @@ __device__ __forceinline__ uint32_t split_mainloop(const KParams &p, const float
     }
     if (nk <= 0) {
         add_low();
-        return tiny;
+        return;
     }
     auto step = [&](auto uc, int t) __attribute__((always_inline)) {
         constexpr int u = decltype(uc)::value, buf = u % 2, slot = (u + 1) % D;
@@ -459,7 +463,6 @@ __device__ __forceinline__ uint32_t split_mainloop(const KParams &p, const float
         if (t + uc < nk) step(uc, t + uc);
     }, std::make_integer_sequence<int, U>{});
     add_low();
-    return tiny;
 }
 
 // The tile again on the fp32 MFMA, operands straight from memory: for the
@@ -779,8 +782,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, 2) void gemm_f32_split(KParams p) 
     // barriers order them before the epilogue reads them)
     __shared__ int ce_t[EPI == EPI_CE ? TM : 1];
     if (EPI == EPI_CE && tid < TM) ce_t[tid] = m0 + tid < M ? p.ce_targets[m0 + tid] : -1;
-    const uint32_t tiny =
-        split_mainloop<TA, TB, CL, WM, WN, MB, WK>(p, A, B, m0, n0, kbeg, kend, lds, acc);
+    split_mainloop<TA, TB, CL, WM, WN, MB, WK>(p, A, B, m0, n0, kbeg, kend, lds, acc);
 
     const int lane = tid & 63, wave = tid % NT >> 6;
     const int wm = wave / WN, wn = wave % WN;
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, 2) void gemm_f32_split(KParams p) 
     }
 
     // ---- what the split does not hold -------------------------------------
-    bool redo = tiny < kTiny;
+    bool redo = false;
     if (first) {
         float nf = 0.0f;  // NaN once any accumulator is not finite
 #pragma unroll
@@ -824,8 +826,11 @@ __global__ __launch_bounds__(WM *WN *WK * 64, 2) void gemm_f32_split(KParams p) 
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) nf = __builtin_fmaf(acc[i][j][r], 0.0f, nf);
-        redo |= !(nf == 0.0f);
+                for (int r = 0; r < 16; ++r) {
+                    acc[i][j][r] *= kUnlift2;
+                    nf = __builtin_fmaf(acc[i][j][r], 0.0f, nf);
+                }
+        redo = !(nf == 0.0f);
     }
     if (EPI == EPI_STORE || EPI == EPI_ACCUM) {
         if (first && __float_as_uint(p.acc_init) != 0) {

@@ -18,9 +18,11 @@ __device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, Is.
     (f(std::integral_constant<int, Is>{}), ...);
 }
 
-// Below this (2 * bits - 1 of 2^-102) a non-zero value's pieces may be
-// subnormal in bf16.
-constexpr uint32_t kTiny = 0x18ffffffu;
+// Operands are lifted by 2^24 before they are split: the lowest bit of any f32
+// is then at least 2^-125, so every piece of every value lies in bf16's normal
+// range, the smallest subnormal's too. Only values from 2^104 on do not fit
+// (they leave infinities), and a product's sums are 2^48 times the true ones.
+constexpr float kLift = 0x1p24f, kUnlift = 0x1p-24f, kUnlift2 = 0x1p-48f;
 
 // (bf16(x), bf16(y)), rounded to nearest even. The empty assembly hides where r
 // comes from: without it the compiler converts x a second time on its own for
@@ -34,11 +36,9 @@ __device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
     return r;
 }
 
-// E values of consecutive k as three pieces of E bf16 each; tiny follows the
-// smallest 2 * |bits| - 1 (zeros wrap to the largest).
+// E values of consecutive k as three pieces of E bf16 each.
 template <int E>
-__device__ __forceinline__ void split_values(const float (&v)[E], uint32_t (&o)[3][E / 2],
-                                             uint32_t &tiny) {
+__device__ __forceinline__ void split_values(const float (&v)[E], uint32_t (&o)[3][E / 2]) {
 #pragma unroll
     for (int i = 0; i < E / 2; ++i) {
         const float x = v[2 * i], y = v[2 * i + 1];
@@ -49,8 +49,23 @@ __device__ __forceinline__ void split_values(const float (&v)[E], uint32_t (&o)[
         o[0][i] = h;
         o[1][i] = m;
         o[2][i] = pack_bf16(sx, sy);
-        tiny = min(tiny, min((__float_as_uint(x) << 1) - 1u, (__float_as_uint(y) << 1) - 1u));
     }
+}
+// Not lifted: tiny follows the smallest 2 * |bits| - 1 (zeros wrap to the largest).
+constexpr uint32_t kTiny = 0x18ffffffu;  // below it pieces may be subnormal
+template <int E>
+__device__ __forceinline__ void split_values(const float (&v)[E], uint32_t (&o)[3][E / 2],
+                                             uint32_t &tiny) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) tiny = min(tiny, (__float_as_uint(v[e]) << 1) - 1u);
+    split_values(v, o);
+}
+template <int E>
+__device__ __forceinline__ void lift_and_split(const float (&v)[E], uint32_t (&o)[3][E / 2]) {
+    float x[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = v[e] * kLift;
+    split_values(x, o);
 }
 
 // An address that is the same in every lane, in scalar registers.

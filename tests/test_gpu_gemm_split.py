@@ -118,6 +118,27 @@ def test_special_values(ctx, what, m, k, n, form):
     assert np.all(np.signbit(acc[m // 4])) and np.all(acc[m // 4] == 0.0)
 
 
+@pytest.mark.parametrize("what,m,k,n", SHAPES, ids=[s[0] for s in SHAPES])
+def test_tiny_values_cost_nothing(ctx, what, m, k, n):
+    # a row of values down to the smallest subnormal, and columns scaled below
+    # 2^-102: the other rows keep their bits, so no tile is formed a second way
+    print(f"\n[gemm split] tiny values, {what}: {m}x{k}x{n}", flush=True)
+    r = np.random.default_rng(m + n)
+    a = r.standard_normal((m, k), dtype=np.float32)
+    b = r.standard_normal((k, n), dtype=np.float32)
+    plain = run(ctx, "nn", a, b)
+    t = a.copy()
+    t[::32] *= np.float32(2.0) ** r.integers(-149, -100, (len(t[::32]), k)).astype(np.float32)
+    out = run(ctx, "nn", t, b)
+    rest = np.arange(m) % 32 != 0
+    assert np.array_equal(out[rest].view(np.uint32), plain[rest].view(np.uint32))
+    check(out, t, b)
+    c = np.ldexp(b, np.where(np.arange(n) % 2, -125, 0)).astype(np.float32)
+    out = run(ctx, "nn", a, c)
+    assert np.array_equal(out[:, ::2].view(np.uint32), plain[:, ::2].view(np.uint32))
+    check(out, a, c)
+
+
 # small products, 32x32 tiles with K split over waves and workgroups: the K
 # around a split's 8 and 16 steps, more than one step per wave, more tiles than
 # CUs, rows that are not 16-byte aligned (summed by fp32 MFMAs: one rounding
