@@ -28,16 +28,23 @@
 // long and a short block of 128 rows on each SIMD (the f32 kernel's way), the
 // long block's wave ran alone most of the time: 136 us at hd128.
 //
-// A wave whose sums are not finite, and every wave of a workgroup that met a
-// value which the pieces cannot hold (in V, or in Q, non-zero below 2^-102),
-// does its strip again in plain f32, one key at a time. Tiny values of K cost
-// a score at most 2^-134 times its query, so they count only beside queries
-// above 2^80, which take the plain way too; probabilities below 2^-110 lose
-// bits that no sum of at least 2^-8 can show.
+// Q, V and P are lifted by 2^24 before they are split (mmh_split.h), so that
+// their small values keep every bit: a probability of 2^-120 beside a value of
+// 2^110 can be a whole output. Q's factor goes into its scale and out of the
+// scores in the exponential's subtraction, V's and P's into the final division;
+// V and P take a multiply per value: 0-2% of the time (B4 H16/8 T1024 hd128 108.6
+// -> 110.9 us, B8 H16/8 T192 hd64 14.2 -> 14.3). (K is split as it is: a piece of it
+// below bf16's normal range moves a score by at most 2^-126 times the query,
+// which no query up to 2^80 shows.)
+//
+// A wave whose sums are not finite (values beyond the lift among them), and
+// every wave of a workgroup with a query above 2^80, does its strip again in
+// plain f32, one key at a time.
 #include "mmh_attention.h"
 #include "mmh_split.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mmh {
 namespace {
@@ -134,9 +141,8 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
     const float *K = p.k + b * p.skb + kvh * p.skh;
     const float *V = p.v + b * p.svb + kvh * p.svh;
 
-    uint32_t tiny = 0xffffffffu;
     // B operand of S^T: the lane's query, head columns 16s + 8*lh .. +7, scaled
-    // into log2 units
+    // into log2 units and lifted
     const float sc = p.scale * kLog2e;
     bf16x8 qp[3][NS];
     float big = 0.0f;
@@ -148,11 +154,11 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
             __builtin_memcpy(v, __builtin_assume_aligned(src + 16 * s, 16), 32);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                v[e] *= sc;
+                v[e] *= sc * kLift;
                 big = fmaxf(big, fabsf(v[e]));
             }
             uint32_t o[3][4];
-            split_values(v, o, tiny);
+            split_values(v, o);
 #pragma unroll
             for (int i = 0; i < 3; ++i) __builtin_memcpy(&qp[i][s], o[i], 16);
         }
@@ -175,7 +181,6 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
     const uint32_t vo = (uint32_t)(16 * vblk + 8 * vsub + 4 * vhalf) * vrow + 4u * (uint32_t)vcol;
     const int kw = kcol / 8 * PK + kkey * 16 + kcol % 8 * 2;
     const int vw = 2 * 3 * SK + (2 * vblk + vhalf) * PV + vcol * 16 + vsub * 8;
-    uint32_t unused = 0xffffffffu;
     // the 64 keys of a step as two tiles of 32
     float st[2][E];
     auto load_k = [&](int step) __attribute__((always_inline)) {
@@ -201,11 +206,12 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
                     float, __builtin_amdgcn_raw_buffer_load_b32(
                                rv, vo + (uint32_t)(step * 64 + 32 * u + 8 * (e >> 2) + (e & 3)) * vrow, 0, 0));
     };
-    auto put = [&](int at, int tile, int piece, uint32_t &small) __attribute__((always_inline)) {
+    auto put = [&](auto lift, int at, int tile, int piece) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             uint32_t o[3][E / 2];
-            split_values(st[u], o, small);
+            if constexpr (decltype(lift)::value) lift_and_split(st[u], o);
+            else split_values(st[u], o);
 #pragma unroll
             for (int i = 0; i < 3; ++i)
                 __builtin_memcpy(__builtin_assume_aligned(lds + u * tile + i * piece + at, 2 * E), o[i], 2 * E);
@@ -251,7 +257,7 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
         float mloc = pv[0];
 #pragma unroll
         for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, pv[r]);
-        mloc = swap_max(mloc);
+        mloc = swap_max(mloc) * kUnlift;
         const bool need = mloc > m_run + 8.0f;  // lazy rescale, as attn_fwd_kernel
         if (__any(need)) {
             const float m_new = need ? mloc : m_run;
@@ -266,7 +272,7 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
         float lsum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            pv[r] = __builtin_amdgcn_exp2f(pv[r] - m_run);
+            pv[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(pv[r], kUnlift, -m_run));
             lsum += pv[r];
         }
         l_run += lsum;  // the lane's own keys; its partner's are added at the end
@@ -278,7 +284,7 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] = pv[8 * kb + e];
             uint32_t w[3][4];
-            split_values(x, w, unused);
+            lift_and_split(x, w);
             bf16x8 ph, pm, pl;
             __builtin_memcpy(&ph, w[0], 16);
             __builtin_memcpy(&pm, w[1], 16);
@@ -311,7 +317,7 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
 #undef MMH_MFMA
 
     load_k(0);
-    put(kw, 3 * SK, SK, unused);
+    put(std::false_type(), kw, 3 * SK, SK);
     load_v(0);
     __syncthreads();
     // A step of 64 keys has two phases with one copy of K and of V in LDS: in
@@ -323,29 +329,29 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
         const int kt = 2 * step + par, next = min(step + 1, nsteps - 1);
         const bool mine = kt < my_tiles;
         if (par) {
-            put(vw, 3 * SV, SV, tiny);
+            put(std::true_type(), vw, 3 * SV, SV);
             load_k(next);
         }
         if (mine) scores(kt);
         if (!par) {
-            put(vw, 3 * SV, SV, tiny);
+            put(std::true_type(), vw, 3 * SV, SV);
             load_k(next);
         }
         __syncthreads();
         if (par) {
-            put(kw, 3 * SK, SK, unused);
+            put(std::false_type(), kw, 3 * SK, SK);
             load_v(next);
         }
         if (mine) apply();
         if (!par) {
-            put(kw, 3 * SK, SK, unused);
+            put(std::false_type(), kw, 3 * SK, SK);
             load_v(next);
         }
         __syncthreads();
     }
 
     // the strip's two halves of the keys meet in LDS, odd tiles' sums first
-    const bool redo_all = __syncthreads_or(tiny < kTiny || big > 0x1p80f);
+    const bool redo_all = __syncthreads_or(big > 0x1p80f * kLift);
     float *sums = reinterpret_cast<float *>(lds) + strip * 32 * OS;
     float2 *ml = reinterpret_cast<float2 *>(lds + 4 * 32 * OS * 4) + strip * 64;
     if (par) {
@@ -386,7 +392,7 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_x3_kernel(AttnP p) {
         return;
     }
     if (qi >= T) return;
-    const float inv = 1.0f / l;
+    const float inv = kUnlift2 / l;
     float *orow = out + (int64_t)qi * p.sot + 4 * lh;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)

@@ -53,10 +53,11 @@ def test_sequence_edges(ctx, B, H, Hkv, hd, T):
     assert err <= 4e-5 * np.abs(v).max()
 
 
+# (T 200 on the split kernel, 150 on the 16-row one)
+@pytest.mark.parametrize("T", [150, 200])
 @pytest.mark.parametrize("B,H,Hkv,hd", [(1, 4, 2, 128), (16, 16, 8, 64)])
-def test_values_the_pieces_do_not_hold(ctx, B, H, Hkv, hd):
-    T = 150
-    print(f"\n[attention split] special values, hd={hd}", flush=True)
+def test_values_the_pieces_do_not_hold(ctx, B, H, Hkv, hd, T):
+    print(f"\n[attention split] special values, hd={hd} T={T}", flush=True)
     q, k, v = inputs(B, H, Hkv, T, hd, 9)
     want = reference(q, k, v)
     # V around 2^-120: its low pieces would be subnormal
@@ -108,3 +109,26 @@ def test_leading_scores_of_minus_infinity(ctx, B, H, Hkv, hd, n):
     # no score but -inf: NaN
     w[..., 0] = big
     assert np.isnan(attend(ctx, w, x, v)[:, :, :n]).all()
+
+
+@pytest.mark.parametrize("B,H,Hkv,hd", [(1, 4, 2, 128), (16, 16, 8, 64)])
+def test_small_probabilities_of_large_values(ctx, B, H, Hkv, hd):
+    # key 0 has the whole weight and values of 0 in all columns but the first,
+    # key 1 a probability of about 2^-n and values of about 2^e: outputs of
+    # those columns are that product alone. Its relative error is the score's (n
+    # in log2 units, rounded with its query's scale: 3 * 2^-24 n ln 2 < 2e-5) and
+    # the product's
+    T = 200
+    print(f"\n[attention split] small probabilities, hd={hd}", flush=True)
+    r = np.random.default_rng(3)
+    for n, e in ((100, 90), (122, 110), (120, 20), (105, 124)):
+        q, k, v = (np.zeros((B, h, T, hd), np.float32) for h in (H, Hkv, Hkv))
+        q[..., 0] = r.uniform(1, 1.02, q.shape[:3])
+        k[:, :, 1, 0] = -n * np.log(2) * np.sqrt(hd)
+        k[:, :, 2:, 0] = -1e5
+        v[:, :, 0, 0] = 1.0
+        v[:, :, 1] = np.ldexp(r.uniform(1, 2, v[:, :, 1].shape), e)
+        got, want = attend(ctx, q, k, v), reference(q, k, v)
+        err = np.abs(got[:, :, 2:, 1:] / want[:, :, 2:, 1:] - 1).max()
+        print(f"  2^-{n} of 2^{e}: max relative error {err:.3g}", flush=True)
+        assert err <= 3e-5
