@@ -29,9 +29,16 @@
 // products they form); B1 16/8 T2048 heads of 128 980 / 590 (256 blocks, one
 // per CU: the longest of them); B1 32/32 T4096 heads of 64 2198 / 1580.
 //
-// A wave with a sum that is not finite, or with a row whose P or dS are all
-// below 2^-90, and every wave of a workgroup that met a non-zero value below 2^-102
-// or staged one above 2^80, does its strip again in plain f32.
+// Every operand is lifted by 2^24 before it is split (mmh_split.h), so that
+// small values keep every bit. P carries its factor into dS; the scores and
+// dP lose theirs in the subtraction that follows, the sums at the end. (Before,
+// the largest and smallest magnitudes were followed to redo such strips: B4
+// 12/12 T1000 heads of 64, with the forward, 205.6 us then, 198.3 now, B1 16/8
+// T2048 heads of 128 598 / 592.)
+//
+// A wave with a sum that is not finite (values beyond the lift among them), and
+// every wave of a workgroup with a log-sum-exp beyond 2^79, whose scores the
+// lift could take to -inf, does its strip again in plain f32.
 #include "mmh_attention.h"
 #include "mmh_split.h"
 
@@ -45,15 +52,12 @@ typedef short shortx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) shortx4 *lds_shortx4;
 
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kSmallRow = 0x1p-90f;
+// log-sum-exps from here on: scores near them may not fit the lift
+constexpr float kLargeLse = 0x1p79f;
 
 __device__ __forceinline__ float swap32_sum(float v) {
     auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(c[0]) + __uint_as_float(c[1]);
-}
-__device__ __forceinline__ float swap32_max(float v) {
-    auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(c[0]), __uint_as_float(c[1]));
 }
 // Over lanes l, l^16, l^32, l^48.
 __device__ __forceinline__ float quad_sum(float v) {
@@ -89,7 +93,7 @@ __device__ __forceinline__ bf16x8 read_tr(const char *lds, int at) {
 
 // Rows of the tile times the stationary operand's pieces w (the lane's row of
 // it, columns 16s + 8*(lane/32) .. +7): out[r] is tile row 8*(r/4) + 4*(lane/32)
-// + r%4 against the lane's.
+// + r%4 against the lane's, lifted twice.
 template <int HD>
 __device__ __forceinline__ void rows_product(const char *tile, const bf16x8 (&w)[3][HD / 16],
                                              float (&out)[16]) {
@@ -116,7 +120,7 @@ __device__ __forceinline__ void rows_product(const char *tile, const bf16x8 (&w)
 }
 
 // acc += columns [32*db0, 32*(db0 + N)) of the tile, transposed, times x (an
-// accumulator-ordered 32-row column per lane).
+// accumulator-ordered 32-row column per lane, lifted).
 template <int HD, int N>
 __device__ __forceinline__ void cols_product(const char *tile, int db0, const float (&x)[16],
                                              floatx16 (&acc)[N]) {
@@ -129,8 +133,8 @@ __device__ __forceinline__ void cols_product(const char *tile, int db0, const fl
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = x[8 * kb + e];
-        uint32_t w[3][4], unused = 0xffffffffu;
-        split_values(v, w, unused);
+        uint32_t w[3][4];
+        split_values(v, w);
         bf16x8 xh, xm, xl;
         __builtin_memcpy(&xh, w[0], 16);
         __builtin_memcpy(&xm, w[1], 16);
@@ -163,19 +167,18 @@ __device__ __forceinline__ void cols_product(const char *tile, int db0, const fl
 }
 #undef MMH_MFMA
 
-// The pieces of a stationary row (times f).
+// The pieces of a stationary row (times f, lifted).
 template <int HD>
-__device__ __forceinline__ void load_pieces(const float *row, float f, bf16x8 (&w)[3][HD / 16],
-                                            uint32_t &tiny) {
+__device__ __forceinline__ void load_pieces(const float *row, float f, bf16x8 (&w)[3][HD / 16]) {
     const float *src = row + 8 * ((threadIdx.x & 63) >> 5);
 #pragma unroll
     for (int s = 0; s < HD / 16; ++s) {
         float v[8];
         __builtin_memcpy(v, __builtin_assume_aligned(src + 16 * s, 16), 32);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] *= f;
+        for (int e = 0; e < 8; ++e) v[e] *= f * kLift;
         uint32_t o[3][4];
-        split_values(v, o, tiny);
+        split_values(v, o);
 #pragma unroll
         for (int i = 0; i < 3; ++i) __builtin_memcpy(&w[i][s], o[i], 16);
     }
@@ -193,14 +196,11 @@ __device__ __forceinline__ void load_values(float (&v)[E], __amdgpu_buffer_rsrc_
     }
 }
 template <int HD>
-__device__ __forceinline__ void put_values(char *tile, const float (&v)[HD / 16], uint32_t &tiny,
-                                           float &big) {
+__device__ __forceinline__ void put_values(char *tile, const float (&v)[HD / 16]) {
     using R = RowTile<HD>;
-#pragma unroll
-    for (int e = 0; e < R::E; ++e) big = fmaxf(big, fabsf(v[e]));
     const int row = threadIdx.x / 16, col = threadIdx.x % 16 * R::E;
     uint32_t o[3][R::E / 2];
-    split_values(v, o, tiny);
+    lift_and_split(v, o);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
         __builtin_memcpy(__builtin_assume_aligned(tile + i * R::PIECE + col / 8 * R::PK + row * 16 + col % 8 * 2,
@@ -208,17 +208,15 @@ __device__ __forceinline__ void put_values(char *tile, const float (&v)[HD / 16]
                          o[i], 2 * R::E);
 }
 
-// Whether the wave's sums have to be formed again: one not finite, or a row
-// whose largest factor is not zero but too small for its pieces.
+// Whether one of the wave's sums is not finite.
 template <int N>
-__device__ __forceinline__ bool wave_redo(const floatx16 (&acc)[N], float largest) {
-    float nf = largest * 0.0f;
+__device__ __forceinline__ bool wave_redo(const floatx16 (&acc)[N]) {
+    float nf = 0.0f;
 #pragma unroll
     for (int i = 0; i < N; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) nf = __builtin_fmaf(acc[i][r], 0.0f, nf);
-    const float big = swap32_max(largest);
-    return __any(!(nf == 0.0f) || (big > 0.0f && big < kSmallRow));
+    return __any(!(nf == 0.0f));
 }
 
 // Strips in plain f32: four lanes (l, l^16, l^32, l^48) share a row, each with a
@@ -336,12 +334,11 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_x3_kernel(BwdP p) {
     const float *dO = p.dout + b * p.sob + head * p.soh;
     const int64_t rows = ((int64_t)b * p.h + head) * T;
 
-    uint32_t tiny = 0xffffffffu;
-    float big = 0.0f;
+    bool large = false;  // a log-sum-exp beyond kLargeLse
     // role 0: the query's row and its log-sum-exp; role 1: dO's row and D
     bf16x8 w[3][HD / 16];
     load_pieces<HD>(role ? dO + (int64_t)qc * p.sot : Q + (int64_t)qc * p.sqt,
-                    role ? 1.0f : p.scale * kLog2e, w, tiny);
+                    role ? 1.0f : p.scale * kLog2e, w);
     float shift;
     if (role) {
         float d = 0.0f;
@@ -355,6 +352,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_x3_kernel(BwdP p) {
         if (lh == 0 && qi < T) p.dvec[rows + qi] = shift;
     } else {
         shift = p.lse[rows + qc];
+        large = fabsf(shift) > kLargeLse;
     }
 
     // thread tid moves E columns of row tid/16 of the K and of the V tile (keys
@@ -368,8 +366,8 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_x3_kernel(BwdP p) {
         load_values(vr, rv, key * svt4 + c);
     };
     auto put = [&](int buf) __attribute__((always_inline)) {
-        put_values<HD>(lds + buf * 2 * R::BYTES, kr, tiny, big);
-        put_values<HD>(lds + buf * 2 * R::BYTES + R::BYTES, vr, tiny, big);
+        put_values<HD>(lds + buf * 2 * R::BYTES, kr);
+        put_values<HD>(lds + buf * 2 * R::BYTES + R::BYTES, vr);
     };
 
     floatx16 acc[N];
@@ -377,7 +375,6 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_x3_kernel(BwdP p) {
     for (int i = 0; i < N; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
-    float largest = 0.0f;
 
     load(0);
     put(0);
@@ -406,10 +403,11 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_x3_kernel(BwdP p) {
                     }
                 }
 #pragma unroll
-                for (int r = 0; r < 16; ++r) x[r] = __builtin_amdgcn_exp2f(x[r] - shift);
+                for (int r = 0; r < 16; ++r)
+                    x[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[r], kUnlift2, -shift)) * kLift;
             } else {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) x[r] -= shift;
+                for (int r = 0; r < 16; ++r) x[r] = __builtin_fmaf(x[r], kUnlift2, -shift);
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -427,16 +425,15 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_x3_kernel(BwdP p) {
                 x[4 * i + 2] *= y.z;
                 x[4 * i + 3] *= y.w;
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) largest = fmaxf(largest, fabsf(x[r]));
             cols_product<HD, N>(kt_lds, role * N, x, acc);
         }
         __syncthreads();
     }
 
-    const bool redo_all = __syncthreads_or(tiny < kTiny || big > 0x1p80f);
-    const bool redo = my_tiles && (wave_redo(acc, largest) || redo_all);
+    const bool redo_all = __syncthreads_or(large);
+    const bool redo = my_tiles && (wave_redo(acc) || redo_all);
     float *dq = p.dq + b * p.sqb + head * p.sqh;
+    const float f = p.scale * kUnlift2;
     if (qi < T) {
         float *row = dq + (int64_t)qi * p.sqt + role * (HD / 2) + 4 * lh;
 #pragma unroll
@@ -444,8 +441,8 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_x3_kernel(BwdP p) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 *reinterpret_cast<float4 *>(row + 32 * i + 8 * j) =
-                    make_float4(acc[i][4 * j] * p.scale, acc[i][4 * j + 1] * p.scale,
-                                acc[i][4 * j + 2] * p.scale, acc[i][4 * j + 3] * p.scale);
+                    make_float4(acc[i][4 * j] * f, acc[i][4 * j + 1] * f, acc[i][4 * j + 2] * f,
+                                acc[i][4 * j + 3] * f);
     }
     // (either wave of the strip redoes all of its columns: both write the same
     // values then, after both have stored theirs)
@@ -487,11 +484,10 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_x3_kernel(BwdP p) {
     const float *dO = p.dout + b * p.sob + head0 * p.soh;
     const int64_t rows = ((int64_t)b * p.h + head0) * T;
 
-    uint32_t tiny = 0xffffffffu;
-    float big = 0.0f;
+    bool large = false;  // a log-sum-exp beyond kLargeLse
     bf16x8 w[3][HD / 16];  // role 0: the key's row of K, role 1: of V
     load_pieces<HD>(role ? V + (int64_t)kc * p.svt : K + (int64_t)kc * p.skt,
-                    role ? 1.0f : p.scale * kLog2e, w, tiny);
+                    role ? 1.0f : p.scale * kLog2e, w);
 
     const __amdgpu_buffer_rsrc_t rq = rsrc_all(Q), rg = rsrc_all(dO);
     const uint32_t sqt4 = 4u * (uint32_t)p.sqt, sot4 = 4u * (uint32_t)p.sot;
@@ -514,9 +510,12 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_x3_kernel(BwdP p) {
         }
     };
     auto put = [&](int buf) __attribute__((always_inline)) {
-        put_values<HD>(lds + buf * BUF, qr, tiny, big);
-        put_values<HD>(lds + buf * BUF + R::BYTES, gr, tiny, big);
-        if (tid < 64) reinterpret_cast<float *>(lds + buf * BUF + 2 * R::BYTES)[tid] = lv;
+        put_values<HD>(lds + buf * BUF, qr);
+        put_values<HD>(lds + buf * BUF + R::BYTES, gr);
+        if (tid < 64) {
+            reinterpret_cast<float *>(lds + buf * BUF + 2 * R::BYTES)[tid] = lv;
+            large |= tid < 32 && fabsf(lv) > kLargeLse;
+        }
     };
 
     floatx16 acc[N];  // role 0: dV^T, role 1: dK^T
@@ -524,7 +523,6 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_x3_kernel(BwdP p) {
     for (int i = 0; i < N; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
-    float largest = 0.0f;
 
     load();
     put(0);
@@ -546,10 +544,10 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_x3_kernel(BwdP p) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float4 y = shift[2 * i + lh];
-                x[4 * i] -= y.x;
-                x[4 * i + 1] -= y.y;
-                x[4 * i + 2] -= y.z;
-                x[4 * i + 3] -= y.w;
+                x[4 * i] = __builtin_fmaf(x[4 * i], kUnlift2, -y.x);
+                x[4 * i + 1] = __builtin_fmaf(x[4 * i + 1], kUnlift2, -y.y);
+                x[4 * i + 2] = __builtin_fmaf(x[4 * i + 2], kUnlift2, -y.z);
+                x[4 * i + 3] = __builtin_fmaf(x[4 * i + 3], kUnlift2, -y.w);
             }
             if (role == 0) {
                 if (!(i0 >= k0 + 31 && i0 + 31 < T)) {
@@ -560,7 +558,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_x3_kernel(BwdP p) {
                     }
                 }
 #pragma unroll
-                for (int r = 0; r < 16; ++r) x[r] = __builtin_amdgcn_exp2f(x[r]);
+                for (int r = 0; r < 16; ++r) x[r] = __builtin_amdgcn_exp2f(x[r]) * kLift;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     ex[strip][i][lane] = make_float4(x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]);
@@ -580,15 +578,13 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_x3_kernel(BwdP p) {
                     x[4 * i + 3] *= y.w;
                 }
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) largest = fmaxf(largest, fabsf(x[r]));
             cols_product<HD, N>(tile + (1 - role) * R::BYTES, 0, x, acc);
         }
         qt = qt + 1 < qt_end ? qt + 1 : qt_first;
         __syncthreads();
     }
 
-    const bool redo_all = __syncthreads_or(tiny < kTiny || big > 0x1p80f);
+    const bool redo_all = __syncthreads_or(large);
     if (k0 >= T) return;
     float *out;
     int64_t out_t;
@@ -599,13 +595,13 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_x3_kernel(BwdP p) {
         out = role ? p.dk + b * p.skb + kvh * p.skh : p.dv + b * p.svb + kvh * p.svh;
         out_t = role ? p.skt : p.svt;
     }
-    if (wave_redo(acc, largest) || redo_all) {
+    if (wave_redo(acc) || redo_all) {
         exact_dkv<HD>(Q, K, V, dO, p.lse + rows, p.dvec + rows, out, p.sqh, p.sqt, p.skt, p.svt,
                       p.soh, p.sot, out_t, p.scale, k0, T, ng, role != 0);
         return;
     }
     if (kj >= T) return;
-    const float f = role ? p.scale : 1.0f;
+    const float f = role ? p.scale * kUnlift2 : kUnlift2;
     float *row = out + (int64_t)kj * out_t + 4 * lh;
 #pragma unroll
     for (int i = 0; i < N; ++i)

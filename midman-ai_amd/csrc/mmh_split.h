@@ -51,15 +51,6 @@ __device__ __forceinline__ void split_values(const float (&v)[E], uint32_t (&o)[
         o[2][i] = pack_bf16(sx, sy);
     }
 }
-// Not lifted: tiny follows the smallest 2 * |bits| - 1 (zeros wrap to the largest).
-constexpr uint32_t kTiny = 0x18ffffffu;  // below it pieces may be subnormal
-template <int E>
-__device__ __forceinline__ void split_values(const float (&v)[E], uint32_t (&o)[3][E / 2],
-                                             uint32_t &tiny) {
-#pragma unroll
-    for (int e = 0; e < E; ++e) tiny = min(tiny, (__float_as_uint(v[e]) << 1) - 1u);
-    split_values(v, o);
-}
 template <int E>
 __device__ __forceinline__ void lift_and_split(const float (&v)[E], uint32_t (&o)[3][E / 2]) {
     float x[E];

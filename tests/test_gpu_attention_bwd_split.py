@@ -100,3 +100,42 @@ def test_values_the_pieces_do_not_hold(ctx, H, Hkv, hd):
     got = backward(ctx, w, k, v, g, 1)
     assert np.isnan(got[0][:, 140]).all() and np.isnan(got[2][:141]).all()
     check(got, want, bound, (others, slice(160, None), slice(160, None)))
+
+
+@pytest.mark.parametrize("H,Hkv,hd", [(8, 8, 128), (16, 16, 64)])
+def test_small_probabilities_of_large_gradients(ctx, H, Hkv, hd):
+    # queries from 2 on give key 0 the whole weight (its values are 0) and key 1
+    # a probability of about 2^-n: key 1's gradients are that probability alone
+    # times one query's gradients of about 2^e. Relative error: the score's (n
+    # in log2 units, a few roundings: 3 * 2^-24 n ln 2 < 2e-5) and the products'
+    T = 210
+    print(f"\n[attention backward split] small probabilities, hd={hd}", flush=True)
+    r = np.random.default_rng(4)
+    for n, e in ((100, 70), (122, 75), (122, 20), (105, 100)):
+        q, k, v, g = (np.zeros((8, h, T, hd), np.float32) for h in (H, Hkv, Hkv, H))
+        q[:, :, 2:, 0] = r.uniform(1, 1.02, q.shape[:2] + (T - 2,))
+        k[:, :, 1, 0] = -n * np.log(2) * np.sqrt(hd)
+        k[:, :, 2:, 0] = -1e5
+        v[:, :, 1:] = r.uniform(1, 2, v[:, :, 1:].shape)
+        g[:, :, 205] = np.ldexp(r.uniform(1, 2, g[:, :, 205].shape), e)
+        dq, dk, dv = backward(ctx, q, k, v, g, 1)
+        (wq, wk, wv), _ = reference(q, k, v, g, 1)
+        err = [np.abs(a / w - 1).max() for a, w in ((dv[1], wv[1]), (dk[:2, 0], wk[:2, 0]),
+                                                    (dq[:, 205, 0], wq[:, 205, 0]))]
+        print(f"  2^-{n} of 2^{e}: max relative errors {err}", flush=True)
+        assert max(err) <= 4e-5
+
+
+@pytest.mark.parametrize("H,Hkv,hd", [(8, 8, 128), (16, 16, 64)])
+def test_scores_beyond_the_lift(ctx, H, Hkv, hd):
+    # all scores the same number of about -2^97: their f32 log-sum-exp is the
+    # score itself, so every probability of the backward is 1
+    T = 210
+    print(f"\n[attention backward split] large scores, hd={hd}", flush=True)
+    q, k, v, g = inputs(8, H, Hkv, T, hd, 5)
+    q[...], k[...] = 0, 0
+    q[..., 0], k[..., 0] = 2.0**50, -(2.0**50)
+    _, _, dv = backward(ctx, q, k, v, g, 1)
+    want = np.cumsum(g[0, 1, ::-1].astype(np.float64), 0)[::-1]
+    size = np.cumsum(np.abs(g[0, 1, ::-1]).astype(np.float64), 0)[::-1]
+    assert np.abs((dv - want) / size).max() <= REL
