@@ -139,6 +139,27 @@ def test_tiny_values_cost_nothing(ctx, what, m, k, n):
     check(out, a, c)
 
 
+@pytest.mark.parametrize("what,m,k,n", SHAPES, ids=[s[0] for s in SHAPES])
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+def test_accumulated_zeros_cost_nothing(ctx, what, m, k, n, form):
+    # rows that are zero over a split's k (padded tokens): its partial sums there
+    # are zero, and what is added to a C of +0 has the bits of the plain product,
+    # so no tile is formed a second way for the sign of a zero that nothing shows
+    print(f"\n[gemm split] accumulated zeros, {what}: {form} {m}x{k}x{n}", flush=True)
+    r = np.random.default_rng(m * n)
+    a = r.standard_normal((m, k), dtype=np.float32)
+    b = r.standard_normal((k, n), dtype=np.float32)
+    a[::2, : k // 4 + 1] = 0
+    a[::2, -(k // 4) :] = 0
+    out = run(ctx, form, a, b, np.zeros((m, n), np.float32))
+    assert np.array_equal(out, run(ctx, form, a, b))
+    # beside a -0 of C a split's zeros keep their sign, and rows of -0 leave it
+    c0 = np.where(np.arange(m)[:, None] % 4 == 0, np.float32(-0.0), np.float32(1.0)) * np.ones((1, n), np.float32)
+    a[::4] = -0.0
+    out = run(ctx, form, a, np.abs(b) + 1, c0)
+    assert np.all(np.signbit(out[::4])) and np.all(out[::4] == 0)
+
+
 # small products, 32x32 tiles with K split over waves and workgroups: the K
 # around a split's 8 and 16 steps, more than one step per wave, more tiles than
 # CUs, rows that are not 16-byte aligned (summed by fp32 MFMAs: one rounding
