@@ -885,6 +885,10 @@ namespace {
 
 int cus_of(const Context &ctx) { return ctx.cu_count > 0 ? ctx.cu_count : 256; }
 
+int64_t big_tiles_of(const GemmDesc &d) {
+    return ((d.m + BM - 1) / BM) * ((d.n + BN - 1) / BN) * d.batch;
+}
+
 // The fp32 MFMA tiles of 64x64: below one 128x128 tile per CU, for products of
 // at most 2^28 multiply-adds (above that the split tiles win: 2048 x 512 x 1024
 // 27.0 -> 20.9 us, 256 x 2048 x 1024 21.2 -> 18.6; at 2^28 the two meet, 4096 x
@@ -892,8 +896,7 @@ int cus_of(const Context &ctx) { return ctx.cu_count > 0 ? ctx.cu_count : 256; }
 // for the ones that take a norm in with their loads (K <= 256), whose own
 // launch costs more than the tiles gain.
 bool use_small(const Context &ctx, const GemmDesc &d) {
-    const int64_t big_tiles = ((d.m + BM - 1) / BM) * ((d.n + BN - 1) / BN) * d.batch;
-    if (big_tiles >= cus_of(ctx)) return false;
+    if (big_tiles_of(d) >= cus_of(ctx)) return false;
     return (d.norm_w && d.k <= 256) || d.m * d.n * d.k <= (int64_t(1) << 28) / d.batch;
 }
 
@@ -1137,6 +1140,7 @@ void gemm(Context &ctx, const GemmDesc &d) {
         if (d.batch != 1) fail(MMH_ERR_ARGUMENT, "gemm: swiglu epilogues take one matrix");
     }
     const int cus = cus_of(ctx);
+    p.libm_exp = big_tiles_of(d) < cus;
     const bool small = use_small(ctx, d);
     const int kind = ksplit_kind(ctx, d);
     const bool ksplit = kind != 0;

@@ -606,7 +606,7 @@ __device__ __forceinline__ void block_epilogue(const KParams &p, const floatx16 
             if (p.aux && col + 1 < N)
                 *reinterpret_cast<float2 *>(p.aux + row * p.ldaux + col) =
                     make_float2(a0[r], a1[r]);
-            if (f < p.swiglu_ff) C[row * p.ldc + f] = __fmul_rn(silu_fast(a0[r]), a1[r]);
+            if (f < p.swiglu_ff) C[row * p.ldc + f] = __fmul_rn(p.libm_exp ? silu_f(a0[r]) : silu_fast(a0[r]), a1[r]);
         }
         return;
     }
@@ -897,11 +897,13 @@ __global__ __launch_bounds__(WM *WN *WK * 64, 2) void gemm_f32_split(KParams p) 
                 const float x0 = col < N ? v0 : -INFINITY, x1 = col + 1 < N ? v1 : -INFINITY;
                 const float mx = half_max32(fmaxf(x0, x1));
                 // exp(z - max) through the hardware's exp2 (no flush concern: the
-                // terms that matter are within a few hundred of 1)
-                const float e = half_sum32(
-                    mx == -INFINITY ? 0.0f
-                                    : __builtin_amdgcn_exp2f((x0 - mx) * kLog2e) +
-                                          __builtin_amdgcn_exp2f((x1 - mx) * kLog2e));
+                // terms that matter are within a few hundred of 1) or libm_exp
+                float e = 0.0f;
+                if (mx != -INFINITY)
+                    e = p.libm_exp ? expf(x0 - mx) + expf(x1 - mx)
+                                   : __builtin_amdgcn_exp2f((x0 - mx) * kLog2e) +
+                                         __builtin_amdgcn_exp2f((x1 - mx) * kLog2e);
+                e = half_sum32(e);
                 if (lr == 0) {
                     ce_m[wn][rl] = mx;
                     ce_s[wn][rl] = e;

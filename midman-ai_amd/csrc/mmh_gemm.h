@@ -45,6 +45,13 @@ struct KParams {
     const int32_t *ce_targets;
     float *ce_part, *ce_zt;
     int ce_tiles;  // 128-column units of a row
+    // Large tiles, the exponentials of EPI_SWIGLU and EPI_CE: libm's (and the IEEE
+    // division) where the grid has less than a 128x128 tile per CU, as the small
+    // kernels have it. The hardware's exp2 of a rounded product, which fuller
+    // grids take, is off by |x| 2^-24 of itself: gates of -60 to -40 give h off by
+    // 3.3e-6, 3.0e-7 by libm's. libm's costs 1-3% of a model's loss there (8 layers
+    // of 768, 512 tokens: 1079 -> 1093 us).
+    int libm_exp;
     // Split K on the 64x64 and 32x32 tiles (tickets set): every split stores
     // its partial tile through to memory and counts itself in tickets[tile];
     // the last split of a tile sums the tile's partials in split order and

@@ -23,7 +23,8 @@ __device__ __forceinline__ float silu_f(float x) {
 // silu through the hardware exp2 and reciprocal (a few ulp from silu_f): 5
 // VALU instructions instead of ~25 for the libm exp and the IEEE division.
 // The VALU's cycles add to the matrix core's on a SIMD, so the large GEMM
-// tiles' epilogue that finishes SwiGLU takes this form.
+// tiles' epilogue that finishes SwiGLU takes this form on grids that fill the
+// chip (KParams::libm_exp).
 __device__ __forceinline__ float silu_fast(float x) {
     const float e = __builtin_amdgcn_exp2f(x * -1.4426950408889634f);
     return x * __builtin_amdgcn_rcpf(1.0f + e);

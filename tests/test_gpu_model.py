@@ -398,3 +398,62 @@ def test_model_errors(ctx):
     with pytest.raises(mh.ArgumentError):
         m.handle = 424242
         m.forward(ids, 1, 8)
+
+
+def one_hot_model(ctx, vocab, ff, wg=None, wu=None, wd=None, head=None):
+    """One layer of width 1024 whose token v enters as 32 in column v, so that
+    every norm scales by exactly 1 and what the weights below hold arrives
+    unrounded: gate and up of token v are rows v of wg and wu. No attention."""
+    d, kv = 1024, 64
+    z = lambda *s: np.zeros(s, np.float32)  # noqa: E731
+    embed = z(vocab, d)
+    embed[np.arange(min(vocab, d)), np.arange(min(vocab, d))] = 32
+    zeros = [z(d, ff), z(d, ff), z(ff, d)]
+    wg, wu, wd = (w if w is not None else o for w, o in zip((wg, wu, wd), zeros))
+    ones = np.ones(d, np.float32)
+    parts = [embed, ones, z(d, d), z(d, kv), z(d, kv), z(d, d), ones / 32, wg, wu, wd, ones / 32, head]
+    w = np.concatenate([np.asarray(p, np.float32).ravel() for p in parts])
+    return mh.Model.from_weights(ctx, [vocab, d, 1, 16, 1, ff, 1024, 10000.0, 1e-30, 0], w)
+
+
+def test_gates_far_below_zero(ctx):
+    # 512 tokens, 128 tiles of 128x128: SwiGLU on the large tiles with libm's
+    # exponential. h of gates in [-60, -40] relative to silu in 64 bits: the
+    # exponential's ulp, four roundings and the final norm's (its mean of 1024
+    # squares): below 1e-6 together
+    print("\n[model] gates in [-60, -40]", flush=True)
+    r = np.random.default_rng(2)
+    d, ff, v = 1024, 2048, 512
+    wg = r.uniform(-60, -40, (d, ff)).astype(np.float32)
+    wu = np.ldexp(r.uniform(1, 2, (d, ff)), 70).astype(np.float32)
+    wd, head = np.zeros((ff, d), np.float32), np.zeros((d, v), np.float32)
+    wd[np.arange(d), np.arange(d)] = 1
+    head[np.arange(v) + v, np.arange(v)] = 1
+    m = one_hot_model(ctx, v, ff, wg, wu, wd, head)
+    got = m.forward(np.arange(v, dtype=np.int32), 1, v)[0]
+    m.close()
+    g, u = wg[:v, :d].astype(np.float64), wu[:v, :d].astype(np.float64)
+    y = g / (1 + np.exp(-g)) * u
+    y[np.arange(v), np.arange(v)] += 32
+    want = y[:, v:] / np.sqrt((y * y).mean(1, keepdims=True)) / 32
+    err = np.abs(got / want - 1).max()
+    print(f"  max relative error {err:.3g}", flush=True)
+    assert err <= 1e-6
+
+
+def test_folded_loss_of_a_small_grid(ctx):
+    # 128 tiles of 128x128: the loss in the head product's epilogue, libm's
+    # exponential. Logits 0 (the target) and 127 of -t, with t where t log2(e) is
+    # rounded the furthest: loss log(1 + 127 exp(-t)), an ulp of the exponential
+    # and two or three roundings of the sum: below 2e-7
+    t = np.linspace(5.6, 6.4, 4001).astype(np.float32)
+    far = (t * np.float32(1.4426950408889634)).astype(np.float64) / 1.4426950408889634 - t
+    for x in (t[far.argmax()], t[far.argmin()]):
+        head = np.zeros((1024, 128), np.float32)
+        head[0, 1:] = -x
+        m = one_hot_model(ctx, 128, 64, head=head)
+        zeros = np.zeros(16 * 1024, np.int32)
+        got, want = m.loss(zeros, zeros, 16, 1024), np.log1p(127 * np.exp(-np.float64(x)))
+        m.close()
+        print(f"\n[model] folded loss {got:.9f} ({got / want - 1:.3g})", flush=True)
+        assert abs(got / want - 1) <= 2e-7
