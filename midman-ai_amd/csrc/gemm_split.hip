@@ -731,23 +731,34 @@ __device__ __forceinline__ void block_epilogue(const KParams &p, const floatx16 
         }
         return;
     }
+    // Single columns (odd rows of C, or the last column). Their reads go out ahead
+    // as well, sixteen at a time, from columns and rows held in range.
+    if (EPI == EPI_ACCUM) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const float *src = R + min(col + j, N - 1);
+            float o[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[r] = src[min(m0 + row_local(r), M - 1) * p.ldc];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int64_t row = m0 + row_local(r);
+                if (row < M && col + j < N)
+                    C[row * p.ldc + col + j] = __fadd_rn(o[r], j ? a1[r] : a0[r]);
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int64_t row = m0 + row_local(r);
         if (row >= M) continue;
         float *dst = C + row * p.ldc + col;
-        const float *src = R + row * p.ldc + col;
-        float v0 = a0[r], v1 = a1[r];
         if (pair) {
-            if (EPI == EPI_ACCUM) {
-                const float2 o = *reinterpret_cast<const float2 *>(src);
-                v0 = __fadd_rn(o.x, v0);
-                v1 = __fadd_rn(o.y, v1);
-            }
-            *reinterpret_cast<float2 *>(dst) = make_float2(v0, v1);
+            *reinterpret_cast<float2 *>(dst) = make_float2(a0[r], a1[r]);
         } else {
-            if (col < N) dst[0] = EPI == EPI_ACCUM ? __fadd_rn(src[0], v0) : v0;
-            if (col + 1 < N) dst[1] = EPI == EPI_ACCUM ? __fadd_rn(src[1], v1) : v1;
+            if (col < N) dst[0] = a0[r];
+            if (col + 1 < N) dst[1] = a1[r];
         }
     }
 }
