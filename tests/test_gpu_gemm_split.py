@@ -160,6 +160,32 @@ def test_accumulated_zeros_cost_nothing(ctx, what, m, k, n, form):
     assert np.all(np.signbit(out[::4])) and np.all(out[::4] == 0)
 
 
+def f32_sums(a, b, block):
+    """The product by f32 sums in order over blocks of k, the blocks' sums in order."""
+    total = None
+    for k0 in range(0, a.shape[1], block):
+        s = np.zeros((a.shape[0], b.shape[1]), np.float32)
+        for k in range(k0, min(k0 + block, a.shape[1])):
+            s += a[:, k, None] * b[k]
+        total = s if total is None else total + s
+    return total
+
+
+# K of a few steps, whose f32 sums round seldom (in order over K here), and shapes
+# of fewer 128x128 tiles than CUs, which had blocks of 32 on the 32x32 tiles
+@pytest.mark.parametrize("m,n,k,block", [(2050, 4100, k, k) for k in (1, 2, 5, 16, 17, 31, 32, 40)]
+                         + [(1472, 1091, 256, 32), (354, 4800, 256, 32), (300, 3456, 320, 32)])
+def test_no_further_off_than_f32_sums(ctx, m, n, k, block):
+    print(f"\n[gemm split] error of {m}x{k}x{n}", flush=True)
+    r = np.random.default_rng(k)
+    a, b = r.standard_normal((m, k), dtype=np.float32), r.standard_normal((k, n), dtype=np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    rel = lambda x: np.linalg.norm(x - want) / np.linalg.norm(want)  # noqa: E731
+    got, ref = rel(run(ctx, "nn", a, b)), rel(f32_sums(a, b, block))
+    print(f"  {got:.3g}, f32 sums {ref:.3g}", flush=True)
+    assert got <= 1.02 * ref
+
+
 # small products, 32x32 tiles with K split over waves and workgroups: the K
 # around a split's 8 and 16 steps, more than one step per wave, more tiles than
 # CUs, rows that are not 16-byte aligned (summed by fp32 MFMAs: one rounding
