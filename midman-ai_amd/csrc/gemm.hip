@@ -894,8 +894,13 @@ int64_t big_tiles_of(const GemmDesc &d) {
 // 27.0 -> 20.9 us, 256 x 2048 x 1024 21.2 -> 18.6; at 2^28 the two meet, 4096 x
 // 512 x 128 10.3 against 13.7 us, 2048 x 128 x 1024 12.9 against 10.0), and
 // for the ones that take a norm in with their loads (K <= 256), whose own
-// launch costs more than the tiles gain.
+// launch costs more than the tiles gain. Also for sums of one step that are added
+// into a C of any size: reading C is their time, which a lone large tile per
+// CU does after its products, several small ones beside each other's (into 960 x
+// 25536 from K 8 55 -> 37 us, 320 x 22528 24 -> 13, 30 shapes 15% on average; from
+// K 33 on it is the large tiles', 0 to 30%).
 bool use_small(const Context &ctx, const GemmDesc &d) {
+    if (d.epi == EPI_ACCUM && d.k <= SBK) return true;
     if (big_tiles_of(d) >= cus_of(ctx)) return false;
     return (d.norm_w && d.k <= 256) || d.m * d.n * d.k <= (int64_t(1) << 28) / d.batch;
 }
@@ -1002,8 +1007,8 @@ constexpr int kMaxTileSplits = 16;
 // G workgroups and q = ceil(G / CUs) on the busiest CU, 16 of K take
 // max(q * alone, G / CUs * full) us (kGemmTiles: a lone workgroup is bound by
 // its own steps, a full chip by its power), a tile's first loads and epilogue
-// about 6 steps more, and split sums a launch and the partials written and
-// read at 4.5 TB/s. Measured constants,
+// some steps more (setup), and split sums a launch and the partials written and
+// read at 3.5 TB/s. Measured constants,
 // f32 TFLOP/s in brackets: 256x256 from 4096 x 2048 x 4096 on (220-228 against
 // 204-206 for 256x128), 256x128 for the grids of 100 to 500 of them (4096 x
 // 2048 x 2048: 197-202; 256x256 150, 128x128 174), 128x128 around one tile per
@@ -1017,12 +1022,17 @@ constexpr int kMaxTileSplits = 16;
 // half of the products measured got slower by up to 10% (919 x 7189 x 490 57 ->
 // 61, 128 x 1664 x 3648 21 -> 23). Past 8 the sums of a split's partials wait
 // on memory once more per four of them, 0.2 us each.
-TilePlan choose_tile(const Context &ctx, const KParams &p, int64_t batch, int epi) {
+// The setups decide where K is a few steps: counted as 6 for every tile, 128x128
+// and 256x256 ones took over from 256x128 (2050 x 64 x 4100 29.5 us, 22.5 so; 7552 x 33
+// x 3763 57 / 51, 2142 x 90 x 1728 27 / 16). Over 260 products of K 33 to 4096 the
+// choice is 0.9% from the best tile of each, 2.9% with 6 for all. (even: 6 for all.)
+TilePlan fastest_tile(const Context &ctx, const KParams &p, int64_t batch, int epi, int first,
+                      bool even) {
     const bool may_split = batch == 1 && (epi == EPI_STORE || epi == EPI_ACCUM) && !p.rope_cos;
     const double cus = cus_of(ctx), ksteps = (double)((p.k + BK - 1) / BK);
     TilePlan best[2];  // of the halvings of K, of the other split counts
     double best_us[2] = {0.0, 0.0};
-    for (int tile = 0; tile < TILE_COUNT; ++tile) {
+    for (int tile = first; tile < TILE_COUNT; ++tile) {
         if (!gemm_tile_takes(p, epi, tile)) continue;
         const GemmTileInfo &t = kGemmTiles[tile];
         const double tiles = (double)((p.m + t.rows - 1) / t.rows) *
@@ -1030,9 +1040,9 @@ TilePlan choose_tile(const Context &ctx, const KParams &p, int64_t batch, int ep
         for (int s = 1; s <= kMaxTileSplits; ++s) {
             // a split keeps 128 of K, as many as its prologue costs
             if (s > 1 && (!may_split || p.k < 128 * s || s * p.m * p.n * 4 > kSplitBytes)) break;
-            const double g = tiles * s;
-            double us = std::max(std::ceil(g / cus) * t.alone, g / cus * t.full) * (ksteps / s + 6.0);
-            if (s > 1) us += 4.0 + (double)(s + 1) * (double)(p.m * p.n) * 4.0 / 4.5e6;
+            const double g = tiles * s, setup = even ? 6.0 : t.setup;
+            double us = std::max(std::ceil(g / cus) * t.alone, g / cus * t.full) * (ksteps / s + setup);
+            if (s > 1) us += 4.0 + (double)(s + 1) * (double)(p.m * p.n) * 4.0 / 3.5e6;
             if (s > 8) us += 0.2 * (s - 8);
             const int fine = s > 8 || (s & (s - 1)) ? 1 : 0;
             if (best_us[fine] == 0.0 || us < best_us[fine]) {
@@ -1043,6 +1053,17 @@ TilePlan choose_tile(const Context &ctx, const KParams &p, int64_t batch, int ep
         }
     }
     return best_us[1] > 0.0 && best_us[1] < 0.96 * best_us[0] ? best[1] : best[0];
+}
+
+// The 256x256 tile's sums round six times per 16 of K, the others' once. It is
+// taken where its steps win, not for its setup: the products of 92 to 480 of K that
+// the setups alone would move to it gain 4-18% over 256x128 and lose a factor of
+// 2.8 in precision.
+TilePlan choose_tile(const Context &ctx, const KParams &p, int64_t batch, int epi) {
+    const TilePlan best = fastest_tile(ctx, p, batch, epi, TILE_256, false);
+    if (best.tile != TILE_256 || fastest_tile(ctx, p, batch, epi, TILE_256, true).tile == TILE_256)
+        return best;
+    return fastest_tile(ctx, p, batch, epi, TILE_256x128, false);
 }
 
 // mmh_gemm_noalloc's contract: which products it takes is stated in terms of a

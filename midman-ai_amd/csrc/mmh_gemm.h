@@ -74,13 +74,13 @@ enum GemmTile : int { TILE_256, TILE_256x128, TILE_128, TILE_128x64, TILE_64, TI
 struct GemmTileInfo {
     int rows, cols;
     // us per 16 of K on an MI355X: a workgroup that has its CU to itself, and
-    // the share of a chip with one on every CU, where its power sets the rate
-    // (choose_tile)
-    float alone, full;
+    // the share of a chip with one on every CU, where its power sets the rate;
+    // and the first loads and the epilogue of a tile in such steps (choose_tile)
+    float alone, full, setup;
 };
 constexpr GemmTileInfo kGemmTiles[TILE_COUNT] = {
-    {256, 256, 1.75f, 2.35f}, {256, 128, 1.0f, 1.29f}, {128, 128, 0.55f, 0.72f},
-    {128, 64, 0.42f, 0.43f},  {64, 64, 0.25f, 0.26f},
+    {256, 256, 1.75f, 2.35f, 7.5f}, {256, 128, 1.0f, 1.29f, 6.0f}, {128, 128, 0.55f, 0.72f, 10.0f},
+    {128, 64, 0.42f, 0.43f, 8.0f},  {64, 64, 0.25f, 0.26f, 14.0f},
 };
 // The tile kernel for p's product in the given form and epilogue; p.tiles_m and
 // p.tiles_n count tiles of the given shape. Splits (grid z) write their sums
