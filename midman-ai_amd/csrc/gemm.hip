@@ -581,7 +581,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_small(KParams p) {
 // staging: lane l takes row (A) or column (B) l%32 and k 16*(l/32) .. +15 of
 // a step, A as four float4 reads of its row and B as sixteen reads that are
 // coalesced across the lanes. The NW partial tiles meet in LDS and are summed
-// in wave order; then wave w applies the epilogue to accumulator registers
+// in pairs; then wave w applies the epilogue to accumulator registers
 // w, w + NW, ... of the sum.
 // NORM: the A rows are RMS-normalised on the way in, as in the small kernel:
 // x * w feeds the MFMAs, the sums of squares of x are gathered per lane and
@@ -602,6 +602,20 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_small(KParams p) {
 // Split K (grid z > 1): each split covers k_per_split values and writes its
 // partial tile; the last split of the tile sums the splits in order and
 // applies the epilogue.
+// N values in pairs, the pairs' sums in pairs and so on: each value is rounded in
+// log2(N) sums instead of up to N (error against 64 bits at 53 x 719 x 3584 1.33e-7
+// -> 1.17e-7; with more splits, before them, 1.21e-7).
+template <int N, class F>
+__device__ __forceinline__ float pair_sum(F &&value, int first = 0) {
+    if constexpr (N == 1) {
+        return value(first);
+    } else {
+        constexpr int H = N > 8 ? 8 : N / 2;
+        const float a = pair_sum<H>(value, first);
+        return __fadd_rn(a, pair_sum<N - H>(value, first + H));
+    }
+}
+
 template <bool TA, bool TB, int EPI, bool NORM, int NW, int MODE>
 __global__ __launch_bounds__(64 * NW) void gemm_f32_mfma_ksplit(KParams p) {
     __shared__ float part[NW][16][64];
@@ -749,9 +763,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_mfma_ksplit(KParams p) {
     for (int i = 0; i < NR; ++i) {
         const int r = wave + i * NW;
         if (r >= 16) break;
-        float v = part[0][r][lane];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) v = __fadd_rn(v, part[w][r][lane]);
+        float v = pair_sum<NW>([&](int w) { return part[w][r][lane]; });
         const int rl = 8 * (r >> 2) + 4 * lk + (r & 3);
         const int64_t row = m0 + rl;
         if (NORM) v = __fmul_rn(v, sm_inv[rl]);

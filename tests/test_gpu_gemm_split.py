@@ -190,6 +190,22 @@ def test_no_further_off_than_f32_sums(ctx, m, n, k, block):
 # around a split's 8 and 16 steps, more than one step per wave, more tiles than
 # CUs, rows that are not 16-byte aligned (summed by fp32 MFMAs: one rounding
 # of at most 2^-24 of the absolute sum per value, and one per split)
+@pytest.mark.parametrize("m,k,n", [(53, 719, 3584), (128, 602, 1984), (1239, 768, 192)])
+def test_small_product_precision(ctx, m, k, n):
+    # f32 sums over the 32 k of a step, the steps' sums in pairs
+    print(f"\n[gemm K split] error of {m}x{k}x{n}", flush=True)
+    r = np.random.default_rng(k)
+    a, b = r.standard_normal((m, k), dtype=np.float32), r.standard_normal((k, n), dtype=np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    steps = [f32_sums(a[:, i:i + 32], b[i:i + 32], 32) for i in range(0, k, 32)]
+    while len(steps) > 1:
+        steps = [x + y for x, y in zip(steps[::2], steps[1::2])] + steps[len(steps) & ~1:]
+    rel = lambda x: np.linalg.norm(x - want) / np.linalg.norm(want)  # noqa: E731
+    got, ref = rel(run(ctx, "nn", a, b)), rel(steps[0])
+    print(f"  {got:.3g}, f32 sums in pairs {ref:.3g}", flush=True)
+    assert got <= 1.05 * ref
+
+
 @pytest.mark.parametrize("m,k,n", [(33, 255, 31), (64, 512, 96), (64, 513, 96), (96, 1024, 96), (128, 2016, 384),
                                    (32, 8192, 32), (2368, 3480, 32), (512, 1600, 320), (1435, 295, 187), (560, 1168, 174),
                                    (92, 1175, 135)])
