@@ -942,26 +942,33 @@ int ksplit_kind(const Context &ctx, const GemmDesc &d) {
 }
 
 // K splits of a kind-2 K-split product: the least estimated time, in ns. A CU
-// holds 16 waves; a round of steps on all of them takes about 4.2 us, on 8
-// waves 3.2 (loads in flight, then the MFMAs); the splits' partials meet in
-// memory for 1.2 us and 0.35 more per split. (It was two workgroups per CU with
-// as few as four steps each: tn 128x384x2048 13.8 us, 8.8 by this estimate,
-// 344x128x2048 13.6 / 8.7, 96x96x1024 8.2 / 6.3, 128x128x8192 18.8 / 13.3,
-// 2048x128x688 (not split any more) 14.5 / 8.7, 128x688x2048 14.5 / 14.4.)
-// uncoalesced: both operands k-major and not 16-byte aligned, read one value
+// holds 16 waves; a round of steps on nw of them takes 0.4 us and 0.185 for
+// each (loads in flight, then the MFMAs), 0.5 where a k-contiguous operand's rows
+// are not 16-byte aligned and come one value at a time; the splits' partials meet in
+// memory for 0.6 us, 0.5 per split and 1.7 per MB. A split keeps four steps.
+// Fitted to 260 products of up to 2^28 multiply-adds with 1 to 32 splits of
+// each: 3% from the best on average. (With eight steps and flatter costs it was 5%,
+// and products of 20 to 30 steps took 10-30% longer than with the two workgroups
+// per CU, whatever their length, before: 41 x 831 x 448 11.1 us, 8.5 so, 100 x 695 x 68
+// 9.9 / 8.3, 81 x 1978 x 192 12.8 / 10.5. Two per CU: tn 128 x 2048 x 384 13.8, 8.8 by the
+// estimate, 16 x 7840 x 341 34.3 / 21.6.)
+// uncoalesced: both operands k-major, not 16-byte aligned, read one value
 // per lane and row: the rows' cache lines bound it, and many small workgroups
-// spread them (nt 574x51x723 10.6 us so, 12.6 by the estimate).
-int ksplit_splits(int cus, int64_t tiles, int64_t ktiles, bool uncoalesced) {
+// spread them (nt 574x51x723 10.6 us so, 12.6 by an estimate).
+int ksplit_splits(int cus, int64_t tiles, int64_t ktiles, int64_t mn, bool unaligned,
+                  bool uncoalesced) {
     int best = 1;
+    if (tiles > Context::kTickets) return best;  // (a counter per tile)
     if (uncoalesced) {
         while (tiles * best < 2 * (int64_t)cus && best < 64 && ktiles / (best * 2) >= 4) best *= 2;
         return best;
     }
     int64_t least = INT64_MAX;
-    for (int s = 1; s <= 64 && (s == 1 || ktiles / s >= 8); s *= 2) {
+    for (int s = 1; s <= 64 && (s == 1 || ktiles / s >= 4); s *= 2) {
         const int64_t steps = (ktiles + s - 1) / s, nw = ksplit_waves(steps);
         const int64_t wgs = cus * (16 / nw), rounds = (tiles * s + wgs - 1) / wgs * ((steps + nw - 1) / nw);
-        const int64_t cost = rounds * (2200 + 125 * nw) + (s > 1 ? 1200 + 350 * s : 0);
+        const int64_t cost = rounds * (400 + (unaligned ? 500 : 185) * nw) +
+                             (s > 1 ? 600 + 500 * s + s * mn * 4 * 17 / 10000 : 0);
         if (cost < least) {
             least = cost;
             best = s;
@@ -1234,7 +1241,9 @@ void gemm(Context &ctx, const GemmDesc &d) {
     if (tiled) {
         splits = plan.splits;
     } else if (kind == 2) {
-        splits = ksplit_splits(cus, tiles, ktiles, !d.ta && d.tb && !(p.vec_a && p.vec_b));
+        splits = ksplit_splits(cus, tiles, ktiles, d.m * d.n,
+                               (!d.ta && !p.vec_a) || (d.tb && !p.vec_b),
+                               !d.ta && d.tb && !(p.vec_a && p.vec_b));
     } else if (!ksplit && d.batch == 1 && d.epi != EPI_SWIGLU && d.epi != EPI_SWIGLU_BWD) {
         // Split only while a split keeps >= 8 steps of 32 (the reduce
         // launch costs about what 8 steps do) and the grid is below a
@@ -1251,9 +1260,10 @@ void gemm(Context &ctx, const GemmDesc &d) {
     p.splits = splits;
     if (splits > 1) {
         // 64x64 and 32x32 tiles: the last split of each tile sums the
-        // partials in split order and applies the epilogue (one launch;
-        // every such grid has fewer tiles than two per CU, far below the
-        // counters); the large tiles: splitk_reduce after the launch
+        // partials in split order and applies the epilogue (one launch; such
+        // grids have less than a 128x128 tile per CU, so at most sixteen
+        // 32x32 tiles: within the counters); the large tiles:
+        // splitk_reduce after the launch
         if (!tiled) {
             p.tickets = d.scratch ? d.scratch_tickets : ctx.tickets;
             if (!p.tickets || tiles > Context::kTickets)
