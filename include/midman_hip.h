@@ -128,9 +128,10 @@ int32_t mmh_gemm_tn(mmh_handle ctx, const float *a, const float *b, float *c, in
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). The same kernels and split choices as the
  * three entry points above, so the same bits; the split-K partials live in a
- * fixed device array per GPU instead of the context's workspace. What it takes
- * is stated for a plan of 128x128 tiles, whose partials may need 16 MiB; a
- * product over that is refused with MMH_ERR_SHAPE before anything runs: a K
+ * fixed device array of 64 MiB per GPU instead of the context's workspace. What it
+ * takes is stated for a plan of 128x128 tiles, whose partials may need 16 MiB
+ * (whatever the kernels' own plan needs, which the array holds); a product over
+ * that is refused with MMH_ERR_SHAPE before anything runs: a K
  * split needs splits x m x n x 4 bytes (chosen only when the output tiles
  * cannot fill the chip; every product of the benchmark sweep fits), the
  * balance of the last tiles 64 KiB per piece (a grid of q x CUs + R tiles cut

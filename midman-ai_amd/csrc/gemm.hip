@@ -1104,8 +1104,9 @@ void check_noalloc(const Context &ctx, const GemmDesc &d) {
         if (splits > 1 && need > limit)
             fail(MMH_ERR_SHAPE, "gemm: the split-K partials of a " + std::to_string(d.m) + " x " +
                                     std::to_string(d.n) + " product (" + std::to_string(splits) +
-                                    " splits) need " + std::to_string(need) +
-                                    " bytes; the scratch holds " + std::to_string(limit));
+                                    " splits of 128x128 tiles) need " + std::to_string(need) +
+                                    " bytes; the scratch holds " + std::to_string(limit) +
+                                    " of such a plan");
         return splits > 1;
     };
     if (big < cus) {
@@ -1138,7 +1139,7 @@ void check_noalloc(const Context &ctx, const GemmDesc &d) {
                                 std::to_string(d.n) + " product (" + std::to_string(r) +
                                 " tiles x " + std::to_string(best_s) + " pieces) need " +
                                 std::to_string(need) + " bytes; the scratch holds " +
-                                std::to_string(limit));
+                                std::to_string(limit) + " of such a plan");
 }
 
 }  // namespace
@@ -1258,6 +1259,12 @@ void gemm(Context &ctx, const GemmDesc &d) {
     p.k_per_split = kt_per * kstep;
     splits = (int)((ktiles + kt_per - 1) / kt_per);
     p.splits = splits;
+    if (d.plan) {
+        d.plan[0] = (int32_t)tile_m;
+        d.plan[1] = (int32_t)tile_n;
+        d.plan[2] = splits;
+        return;
+    }
     if (splits > 1) {
         // 64x64 and 32x32 tiles: the last split of each tile sums the
         // partials in split order and applies the epilogue (one launch; such

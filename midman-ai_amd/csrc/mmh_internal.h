@@ -163,6 +163,8 @@ struct GemmDesc {
     // With scratch: kTickets zeroed tile counters for the in-kernel split
     // reduction (null: the context's own).
     int32_t *scratch_tickets = nullptr;
+    // Receives rows and columns of a tile and the K splits; nothing runs then.
+    int32_t *plan = nullptr;
     // EPI_ACCUM with the GEMM seam's rule (kernels.rs:48, C += A.B): C's own
     // value starts the sum. Without it EPI_ACCUM is a residual add of a fresh
     // product (block.rs:79-80: x + matmul(..), the product summed from +0).

@@ -270,7 +270,8 @@ int32_t mmh_randn(uint64_t seed, float std_, float *out_host, int64_t n) {
 // ---- GEMM seam ----------------------------------------------------------------
 
 static int32_t gemm_entry(mmh_handle ctx, const float *a, const float *b, float *c, int64_t m,
-                          int64_t k, int64_t n, int32_t accumulate, bool ta, bool tb) {
+                          int64_t k, int64_t n, int32_t accumulate, bool ta, bool tb,
+                          int32_t *plan = nullptr) {
     return guard([&] {
         Context &cx = context(ctx);
         need(a, "a");
@@ -293,9 +294,18 @@ static int32_t gemm_entry(mmh_handle ctx, const float *a, const float *b, float 
         d.ldc = n;
         d.epi = accumulate ? EPI_ACCUM : EPI_STORE;
         d.accumulate_into_c = accumulate != 0;
+        d.plan = plan;
         gemm(cx, d);
         return MMH_OK;
     });
+}
+
+// For the tests, not part of the C ABI: the tile (rows, columns) and the K splits
+// that mmh_gemm_nn, _nt or _tn would take for these operands.
+int32_t mmh_test_gemm_plan(mmh_handle ctx, int32_t form, const float *a, const float *b, float *c,
+                           int64_t m, int64_t k, int64_t n, int32_t accumulate, int32_t *plan) {
+    return gemm_entry(ctx, a, b, c, m, k, n, accumulate, form == MMH_GEMM_TN, form == MMH_GEMM_NT,
+                      plan);
 }
 
 int32_t mmh_gemm_nn(mmh_handle ctx, const float *a, const float *b, float *c, int64_t m,

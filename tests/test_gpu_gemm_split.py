@@ -7,6 +7,8 @@ group of 16 k, six groups per 16 k, each below 2^-23 S (it may truncate); a K
 split adds at most 16 partials, a rounding of 2^-24 each. So |err| <=
 (6 * ceil(k / 16) + 16) * 2^-23 * S.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -14,21 +16,55 @@ import midman_hip as mh
 
 pytestmark = pytest.mark.gpu
 
-# (m, k, n) with row, column and K remainders; which tile the choice in
-# gemm.hip gives each on 256 CUs
-SHAPES = [
-    ("256x256, K tail", 3900, 100, 4000),
-    ("256x128, whole steps", 2050, 64, 4100),
-    ("256x128 in 2 splits", 1000, 2050, 4100),
-    ("128x128, 2 wave groups, odd step and tail", 1000, 777, 3071),
-    ("128x128 in splits", 1003, 1517, 770),
-    ("128x64, an odd step", 2000, 528, 1001),
-    ("64x64, 4 wave groups, 3 odd steps and a tail", 1030, 569, 515),
-    ("64x64 in splits", 300, 5003, 301),
-    ("128x128 in 3 splits", 767, 1598, 1373),
-    ("64x64 in 16 splits", 130, 9001, 257),
-    ("64x64, fewer whole steps than wave groups", 2300, 50, 2301),
+# (m, k, n) with row, column and K remainders, and the tile and K splits that
+# the choice in gemm.hip gives each on 256 CUs (test_plans holds it to that)
+PLANS = [
+    ("256x128, K tail", 3900, 100, 4000, 1),
+    ("256x128, whole steps", 2050, 64, 4100, 1),
+    ("256x256 in 3 splits", 1000, 2050, 4100, 3),
+    ("128x128, 2 wave groups, odd step and tail", 1000, 777, 3071, 1),
+    ("64x64, 4 wave groups, 2 odd steps and a tail", 1003, 1517, 770, 1),
+    ("128x64, an odd step", 2000, 528, 1001, 1),
+    ("64x64, 4 wave groups, 3 odd steps and a tail", 1030, 569, 515, 1),
+    ("64x64 in 10 splits", 300, 5003, 301, 10),
+    ("128x128 in 3 splits", 767, 1598, 1373, 3),
+    ("64x64 in 16 splits", 130, 9001, 257, 16),
+    ("256x128, few steps and a tail", 2300, 50, 2301, 1),
+    ("256x256, K tail", 3344, 66, 3105, 1),
+    ("256x128 in 11 splits", 134, 3670, 2208, 11),
+    ("128x64 in 6 splits", 341, 899, 876, 6),
+    ("128x64, fewer whole steps than wave groups", 32768, 31, 60, 1),
 ]
+SHAPES = [p[:4] for p in PLANS]
+# small products, 32x32 tiles with K split over waves and workgroups: the K
+# around a split's 8 and 16 steps, more than one step per wave, more tiles than
+# CUs, rows that are not 16-byte aligned (summed by fp32 MFMAs: one rounding
+# of at most 2^-24 of the absolute sum per value, and one per split)
+SMALL = [(33, 255, 31), (64, 512, 96), (64, 513, 96), (96, 1024, 96), (128, 2016, 384),
+         (32, 8192, 32), (2368, 3480, 32), (512, 1600, 320), (1435, 295, 187), (560, 1168, 174),
+         (92, 1175, 135)]
+
+
+def plan(ctx, form, m, k, n, accumulate=0):
+    """(rows, columns, K splits) of the tiles a product of 16-byte aligned operands takes."""
+    out, x = (ctypes.c_int32 * 3)(), ctx.empty((4,))
+    at = ctypes.c_void_p(x.ptr)
+    mh.check(mh.lib().mmh_test_gemm_plan(
+        ctypes.c_int64(ctx.handle), {"nn": 0, "nt": 1, "tn": 2}[form], at, at, at, ctypes.c_int64(m),
+        ctypes.c_int64(k), ctypes.c_int64(n), accumulate, out))
+    x.free()
+    return tuple(out)
+
+
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+def test_plans(ctx, form):
+    if ctx.device_info()[1] != 256:
+        pytest.skip("the plans are those of 256 CUs")
+    for what, m, k, n, splits in PLANS:
+        rows, cols = (int(x) for x in what.replace(",", " ").split()[0].split("x"))
+        assert plan(ctx, form, m, k, n) == (rows, cols, splits), what
+        assert plan(ctx, form, m, k, n, 1)[:2] == ((rows, cols) if k > 32 else (64, 64)), what
+    assert all(plan(ctx, form, m, k, n)[:2] == (32, 32) for m, k, n in SMALL)
 
 
 def run(ctx, form, a, b, c0=None):
@@ -139,7 +175,8 @@ def test_tiny_values_cost_nothing(ctx, what, m, k, n):
     check(out, a, c)
 
 
-@pytest.mark.parametrize("what,m,k,n", SHAPES, ids=[s[0] for s in SHAPES])
+# (a K of one step of 32 accumulates on the fp32 64x64 tiles)
+@pytest.mark.parametrize("what,m,k,n", [s for s in SHAPES if s[2] > 32], ids=[s[0] for s in SHAPES if s[2] > 32])
 @pytest.mark.parametrize("form", ["nn", "nt", "tn"])
 def test_accumulated_zeros_cost_nothing(ctx, what, m, k, n, form):
     # rows that are zero over a split's k (padded tokens): its partial sums there
@@ -186,10 +223,6 @@ def test_no_further_off_than_f32_sums(ctx, m, n, k, block):
     assert got <= 1.02 * ref
 
 
-# small products, 32x32 tiles with K split over waves and workgroups: the K
-# around a split's 8 and 16 steps, more than one step per wave, more tiles than
-# CUs, rows that are not 16-byte aligned (summed by fp32 MFMAs: one rounding
-# of at most 2^-24 of the absolute sum per value, and one per split)
 @pytest.mark.parametrize("m,k,n", [(53, 719, 3584), (128, 602, 1984), (1239, 768, 192)])
 def test_small_product_precision(ctx, m, k, n):
     # f32 sums over the 32 k of a step, the steps' sums in pairs
@@ -206,9 +239,7 @@ def test_small_product_precision(ctx, m, k, n):
     assert got <= 1.05 * ref
 
 
-@pytest.mark.parametrize("m,k,n", [(33, 255, 31), (64, 512, 96), (64, 513, 96), (96, 1024, 96), (128, 2016, 384),
-                                   (32, 8192, 32), (2368, 3480, 32), (512, 1600, 320), (1435, 295, 187), (560, 1168, 174),
-                                   (92, 1175, 135)])
+@pytest.mark.parametrize("m,k,n", SMALL)
 @pytest.mark.parametrize("form", ["nn", "nt", "tn"])
 def test_small_product_splits(ctx, m, k, n, form):
     print(f"\n[gemm K split] {form} {m}x{k}x{n}", flush=True)
