@@ -20,7 +20,7 @@
 // partials are summed in split order, so the result is deterministic: on the
 // 64x64 and 32x32 tiles by the last split of each tile (the splits store
 // their partial through to memory and count themselves in a per-tile
-// counter), on the 128x128 tiles by a second kernel.
+// counter), on the large tiles by a second kernel.
 #include "mmh_gemm.h"
 
 #include <algorithm>
@@ -241,7 +241,7 @@ __device__ __forceinline__ void small_mainloop(const KParams &p, const float *__
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int idx = tid + 256 * i;
-            // padding: A -0, B +0, so a padded product is -0 (see load_a_edge)
+            // padding: A -0, B +0, so a padded product is -0, the identity of addition
             float4 v = make_float4(-0.f, -0.f, -0.f, -0.f), w = make_float4(0.f, 0.f, 0.f, 0.f);
             if (!TA) {
                 const int64_t gm = m0 + (idx >> 3), gk = k0 + (idx & 7) * 4;
@@ -1269,7 +1269,7 @@ void gemm(Context &ctx, const GemmDesc &d) {
         // 64x64 and 32x32 tiles: the last split of each tile sums the
         // partials in split order and applies the epilogue (one launch; such
         // grids have less than a 128x128 tile per CU, so at most sixteen
-        // 32x32 tiles: within the counters); the large tiles:
+        // 32x32 tiles per CU: within the counters); the large tiles:
         // splitk_reduce after the launch
         if (!tiled) {
             p.tickets = d.scratch ? d.scratch_tickets : ctx.tickets;

@@ -12,6 +12,7 @@ import pytest
 
 import midman_hip as mh
 import mm_oracle as O
+from test_gpu_gemm_split import plan
 
 pytestmark = pytest.mark.gpu
 
@@ -77,16 +78,15 @@ def test_sweep_forward_and_backward(ctx, k, n):
 @pytest.mark.parametrize("m,k,n", [(1, 1, 1), (3, 5, 7), (12, 16, 32), (33, 17, 65),
                                    (129, 250, 131), (64, 4097, 40), (300, 8, 1000),
                                    (2048, 128, 4096),
-                                   # the 128x128 kernel's load ring (3 slots, unrolled by 6)
-                                   # with 1, 3, 6 and 7 K-tiles, the last with ragged edges
+                                   # the 256x128 tiles with 1, 3, 6 and 7 steps of K, the
+                                   # last with ragged edges
                                    (2048, 16, 4096), (2048, 48, 4096), (2048, 96, 4096),
                                    (2050, 112, 4100),
                                    # short-K shapes of the tiny preset and its edges
                                    (2048, 128, 384), (2048, 352, 128), (2047, 480, 97),
                                    (2000, 481, 50), (65, 33, 700),
-                                   # 384 and 448 tiles of 128x128 on 256 CUs: the last
-                                   # 128 / 192 run as 2 / 4 K-pieces + tail_reduce
-                                   # (ragged edges and a short last piece in the first)
+                                   # grids of one and a half 256x128 tiles per CU, with
+                                   # ragged edges and a short last step in the first
                                    (3000, 1000, 2000), (3584, 1024, 2048)])
 @pytest.mark.parametrize("form", ["nn", "nt", "tn"])
 def test_ragged_shapes_and_accumulate(ctx, m, k, n, form):
@@ -112,22 +112,31 @@ GUARD = 0x7FC0DEAD  # the reference's guard value (kernels_avx.rs:374)
 MIN_POSITIVE = np.float32(1.17549435e-38)
 
 # Shapes that route the seam to each kernel path (gemm.hip's dispatch on a
-# 256-CU MI355X): the 128x128 kernel with interior and edge tiles; the 64x64
-# kernel with a partial K step; the 32x32 K-split kernel in one workgroup
-# (nn; nt and tn of this shape split K across two workgroups); the K-split
-# kernel split across workgroups plus splitk_reduce; the 128x128 kernel split
-# along K plus splitk_reduce.
+# 256-CU MI355X, held to it below): the large tiles with interior and edge tiles
+# and a K tail; the same split along K, summed by splitk_reduce; the 32x32
+# K-split kernel in one workgroup and split across workgroups, summed by each
+# tile's last split; the 64x64 kernel, which a sum of one step into a C takes.
 SPECIAL_PATHS = [
-    ("128x128 tiles, interior and edges", 1100, 48, 4100),
-    ("64x64 tiles, partial K step", 2048, 500, 1024),
-    # K beyond 1024 on the 64x64 tiles (at most 2^29 multiply-adds): 4 splits
-    # of 16 K-steps, the last one short, summed by each tile's last split
-    ("64x64 tiles, K 2000 in 4 splits summed by the last split", 256, 2000, 1024),
+    ("256x128 tiles, interior and edges", 1100, 48, 4100),
+    ("128x64 tiles, a K tail", 2048, 500, 1024),
+    ("128x64 tiles, K 2000 in 8 splits", 256, 2000, 1024),
     ("32x32 K-split tiles", 2048, 344, 128),
-    ("32x32 K-split over 8 workgroups + reduce", 256, 2048, 256),
-    ("128x128 split 8 ways along K + reduce", 1024, 8192, 1024),
-    ("128x128 whole tiles + K-pieces of the last tiles + tail_reduce", 3000, 1000, 2000),
+    ("32x32 K-split tiles in 4 splits", 256, 2048, 256),
+    ("256x128 tiles in 8 splits", 1024, 8192, 1024),
+    ("256x128 tiles, one and a half per CU", 3000, 1000, 2000),
+    ("256x128 tiles, 64x64 when accumulating", 4100, 30, 1030),
 ]
+
+
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+def test_special_paths_are_those_named(ctx, form):
+    if ctx.device_info()[1] != 256:
+        pytest.skip("the plans are those of 256 CUs")
+    for what, m, k, n in SPECIAL_PATHS:
+        rows, cols = (int(x) for x in what.split()[0].split("x"))
+        splits = int(what.split(" in ")[1].split()[0]) if " in " in what else 1
+        assert plan(ctx, form, m, k, n) == (rows, cols, splits), what
+        assert plan(ctx, form, m, k, n, 1)[:2] == ((64, 64) if k == 30 else (rows, cols)), what
 
 
 def special_operands(m, k, n, seed):

@@ -44,14 +44,13 @@ def operands(form, m, k, n, seed):
     # dB = A^T dC of the benchmark sweep (a 2048-long reduction into 256 x 256:
     # split across workgroups), then a smaller split product
     ("tn", (256, 2048, 256), (128, 1024, 96)),
-    # the 128x128 kernel split along K (16 tiles), then the K-split kernel
+    # 128x64 tiles in 8 splits summed by a second kernel, then the K-split kernel
     ("nn", (512, 8192, 512), (300, 2000, 200)),
     ("nt", (256, 4096, 1024), (64, 512, 64)),
-    # the sweep's largest partials (16 MiB: dB 4096 x 256 from 2048 rows, 4
-    # splits), then the smallest sweep dB
+    # the sweep's tallest dB (4096 x 256 from 2048 rows: 64x64 tiles, whole),
+    # then the smallest, split
     ("tn", (4096, 2048, 256), (256, 2048, 256)),
-    # the sweep's 1 GFLOP dB products: 64x64 tiles, 4 splits summed by each
-    # tile's last split (the counters in the static set)
+    # the sweep's 1 GFLOP dB products: 128x64 tiles in 8 splits
     ("tn", (256, 2048, 1024), (1024, 2048, 256)),
 ])
 @pytest.mark.parametrize("accumulate", [False, True])
@@ -71,9 +70,9 @@ def test_noalloc_unsplit_product_and_errors(ctx):
     want = run(ctx, "alloc", "nn", a, b, c0, 2048, 256, 4096, False)
     got = run(ctx, "noalloc", "nn", a, b, c0, 2048, 256, 4096, False)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
-    # partials over the 16 MiB array: 1152 x 2048 (144 tiles of 128 x 128)
-    # from a 2048-long reduction splits 2 ways, 18.9 MB of partials; refused,
-    # the output untouched
+    # partials over the stated 16 MiB: 1152 x 2048 (144 tiles of 128 x 128)
+    # from a 2048-long reduction, 2 splits of 128 x 128 tiles, 18.9 MB of
+    # partials; refused, the output untouched
     m, k, n = 1152, 2048, 2048
     A, B = ctx.empty((m, k)), ctx.empty((k, n))
     C = ctx.to_device(np.full((m, n), 3.0, np.float32))
@@ -92,10 +91,10 @@ def test_noalloc_unsplit_product_and_errors(ctx):
 
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_noalloc_tail_balanced_product(ctx, accumulate):
-    # tiles = CUs + 16 of 128 x 128 (2048 columns): the last 16 tiles are cut
-    # along K into 8 pieces (8 MiB of partials, inside the array) and summed
-    # in piece order by tail_reduce, on both entry points; then a smaller
-    # split product through the same array
+    # tiles = CUs + 16 of 128 x 128 (2048 columns), whose last 16 cut along K
+    # into 8 pieces would need 8 MiB: taken; the kernels run 256x256 tiles in
+    # 3 splits on both entry points; then a smaller split product through the
+    # same array
     _, cus = ctx.device_info()
     m, k, n = 128 * (cus // 16 + 1), 2048, 2048
     print(f"\n[gemm_noalloc tail] nn {m}x{k}x{n} ({cus} CUs) accumulate={accumulate}", flush=True)
@@ -107,9 +106,9 @@ def test_noalloc_tail_balanced_product(ctx, accumulate):
 
 
 def test_noalloc_refuses_tail_pieces_over_the_array(ctx):
-    # tiles = CUs + (CUs / 2 + 1): the tail takes 8 pieces per tile, about
-    # 66 MiB of partials on 256 CUs: the allocating entry point runs it, the
-    # no-alloc one refuses it (never a different split) and leaves C alone
+    # tiles = CUs + (CUs / 2 + 1) of 128 x 128: 8 pieces per tile of the tail
+    # would need about 66 MiB of partials on 256 CUs: the allocating entry point
+    # runs it, the no-alloc one refuses it and leaves C alone
     _, cus = ctx.device_info()
     tiles_n = 11
     rows = -(-(cus + cus // 2 + 1) // tiles_n)
