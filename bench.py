@@ -40,9 +40,9 @@ PEAK_SPLIT_F32_TFLOPS = 419.4
 # rocprofv3 passes over this same bench (--pmc FETCH_SIZE, then --pmc
 # WRITE_SIZE, --steps 1 --warmup 0 --train-steps 0 --copy-probe), each scaled by
 # what the counter reads for the add kernel's known traffic (FETCH x 2.0,
-# WRITE x 1.0): (28,757,482 + 7,432,481) KiB over 81 launches. The counters
+# WRITE x 1.0): (29,699,835 + 6,295,171) KiB over 81 launches. The counters
 # cannot be read from inside this process; see profiles/large_forward_hbm_traffic.md.
-GEMM_TRAFFIC_BYTES_PER_LAUNCH = 457.5e6
+GEMM_TRAFFIC_BYTES_PER_LAUNCH = 455.0e6
 
 
 def log(msg):

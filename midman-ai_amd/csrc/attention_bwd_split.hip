@@ -23,7 +23,7 @@
 //
 // What bounds it: the matrix cores at the clock their power leaves them, then
 // the VALU: per 32x32 tile and wave at heads of 128, 96 MFMAs (dkv) or 72 (dq)
-// beside about 350 VALU instructions. Whole backward with its forward, fp32
+// beside about 330 VALU instructions. Whole backward with its forward, fp32
 // matrix cores against this: B4 12/12 T1000 heads of 64 308 / 197 us; B4 16/8
 // T1024 heads of 128 604 / 457 (these kernels 344: 175 TFLOP/s of the seven
 // products they form); B1 16/8 T2048 heads of 128 980 / 590 (256 blocks, one

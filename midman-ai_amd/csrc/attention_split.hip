@@ -19,8 +19,8 @@
 // attention.hip's.
 //
 // What bounds it: the chip's power and the VALU. For 32 queries x 32 keys at
-// heads of 128 a wave runs 96 MFMAs beside about 590 VALU instructions (280
-// for its share of K's and V's pieces, 140 for P's, the softmax) and reads 48
+// heads of 128 a wave runs 96 MFMAs beside about 540 VALU instructions (260
+// for its share of K's and V's pieces, 150 for P's, the softmax) and reads 48
 // KB of LDS; matrix cores and VALU are each busy about 45% of the cycles.
 // Measured (f32 MFMA kernel before -> now): B4 H16/8 T1024 hd128 159 -> 120-124
 // us = 140 TFLOP/s, B1 H16/8 T2048 hd128 264 -> 136-146, B4 H12 T1000 hd64 82 ->
