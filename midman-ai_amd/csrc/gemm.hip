@@ -942,16 +942,17 @@ int ksplit_kind(const Context &ctx, const GemmDesc &d) {
 }
 
 // K splits of a kind-2 K-split product: the least estimated time, in ns. A CU
-// holds 16 waves; a round of steps on nw of them takes 0.4 us and 0.185 for
-// each (loads in flight, then the MFMAs), 0.5 where a k-contiguous operand's rows
-// are not 16-byte aligned and come one value at a time; the splits' partials meet in
-// memory for 0.6 us, 0.5 per split and 1.7 per MB. A split keeps four steps.
-// Fitted to 260 products of up to 2^28 multiply-adds with 1 to 32 splits of
-// each: 3% from the best on average. (With eight steps and flatter costs it was 5%,
-// and products of 20 to 30 steps took 10-30% longer than with the two workgroups
-// per CU, whatever their length, before: 41 x 831 x 448 11.1 us, 8.5 so, 100 x 695 x 68
-// 9.9 / 8.3, 81 x 1978 x 192 12.8 / 10.5. Two per CU: tn 128 x 2048 x 384 13.8, 8.8 by the
-// estimate, 16 x 7840 x 341 34.3 / 21.6.)
+// holds 16 waves; a round of workgroups costs 2.7 us to start, sum and store and
+// its nw waves 0.3 and 0.27 each for every step they take one after another
+// (loads in flight, then the MFMAs); 4.2 and 0.5 where a k-contiguous operand's rows
+// are not 16-byte aligned and come one value at a time. The splits' partials meet in
+// memory for 1.1 us, 0.75 per split and 2 per MB. A split keeps four steps.
+// Fitted to 680 products of up to 2^28 multiply-adds with 1 to 32 splits of
+// each: 2.1% from the best on average. (Eight steps a split and one cost per step:
+// 4.0%, and products of 20 to 30 steps took 10-30% longer than with two workgroups
+// per CU, whatever their length, before that: 41 x 831 x 448 11.1 us, 8.5 so, 100 x 695
+// x 68 9.9 / 8.3, 81 x 1978 x 192 12.8 / 10.5. Two per CU: tn 128 x 2048 x 384 13.8, 8.8
+// by the estimate, 16 x 7840 x 341 34.3 / 21.6.)
 // uncoalesced: both operands k-major, not 16-byte aligned, read one value
 // per lane and row: the rows' cache lines bound it, and many small workgroups
 // spread them (nt 574x51x723 10.6 us so, 12.6 by an estimate).
@@ -966,9 +967,10 @@ int ksplit_splits(int cus, int64_t tiles, int64_t ktiles, int64_t mn, bool unali
     int64_t least = INT64_MAX;
     for (int s = 1; s <= 64 && (s == 1 || ktiles / s >= 4); s *= 2) {
         const int64_t steps = (ktiles + s - 1) / s, nw = ksplit_waves(steps);
-        const int64_t wgs = cus * (16 / nw), rounds = (tiles * s + wgs - 1) / wgs * ((steps + nw - 1) / nw);
-        const int64_t cost = rounds * (400 + (unaligned ? 500 : 185) * nw) +
-                             (s > 1 ? 600 + 500 * s + s * mn * 4 * 17 / 10000 : 0);
+        const int64_t wgs = cus * (16 / nw), rounds = (tiles * s + wgs - 1) / wgs;
+        const int64_t start = unaligned ? 4200 : 2700, wave = unaligned ? 500 : 270;
+        const int64_t cost = rounds * (start + (steps + nw - 1) / nw * (300 + wave * nw)) +
+                             (s > 1 ? 1100 + 750 * s + s * mn * 8 / 1000 : 0);
         if (cost < least) {
             least = cost;
             best = s;
